@@ -288,15 +288,30 @@ struct MfMain {
       }
     };
 #pragma unroll
-    for (int d = 0; d < D; ++d) issue(buf[d], d);
+    for (int d = 0; d < D; ++d) {
+      issue(buf[d], d);
+      if constexpr (VEC) __builtin_amdgcn_sched_barrier(0);  // the slots' loads in slot order
+    }
     hook();
-    for (int64_t base = 0; base < nseg; base += D) {
+    // Whole rounds without a branch inside, then the last 1..D segments without loads: a branch around a slot's MFMAs
+    // made every round wait for all loads in flight, its own included (2048 x 2560 bf16 at one row: see the launch menu).
+    int64_t base = 0;
+    if (nseg > D) {
+      do {
 #pragma unroll
-      for (int d = 0; d < D; ++d) {
-        if (base + d < nseg) compute_slot(buf[d], xs, s_first + (base + d) * stride, acc);
-        if (d == 0 && base == 0) first();
-        issue(buf[d], base + d + D);
-      }
+        for (int d = 0; d < D; ++d) {
+          compute_slot(buf[d], xs, s_first + (base + d) * stride, acc);
+          if (d == 0 && base == 0) first();
+          issue(buf[d], base + d + D);
+          if constexpr (VEC) __builtin_amdgcn_sched_barrier(0);
+        }
+        base += D;
+      } while (base + D < nseg);
+    }
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      if (base + d < nseg) compute_slot(buf[d], xs, s_first + (base + d) * stride, acc);
+      if (d == 0 && base == 0) first();
     }
   }
 };
