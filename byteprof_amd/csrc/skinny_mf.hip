@@ -10,6 +10,7 @@
 
 #define BP_MF_INSTANTIATE
 #include "skinny_mf_kernel.h"
+#include "skinny_wide.h"
 
 namespace bp {
 
@@ -44,6 +45,16 @@ int mf_row_groups(int xstage) {
 }
 
 int mf_blocks(int64_t M) { return M <= 8 ? 1 : M <= 16 ? 2 : M <= 32 ? 4 : 8; }
+
+// The plans a vector launch takes: rb 1, 2, 4 (4 up to 16 rows), waves 1, 2, 4, 8; staged activations up to 16 rows; row
+// groups with staged activations at 9..16 rows, waves x groups <= 16. The sums are the same whichever kernel runs them.
+bool mf_menu(int wkind, int mb, int rb, int waves, bool xl, int wr) {
+  if (wkind != kBf16 && wkind != kInt8) return false;
+  if ((rb != 1 && rb != 2 && !(rb == 4 && mb <= 2)) || (waves != 1 && waves != 2 && waves != 4 && waves != 8))
+    return false;
+  if (xl && mb > 2) return false;
+  return wr == 1 || (xl && mb == 2 && waves >= 2 && waves * wr <= 16);
+}
 
 int mf_status() {
   const hipError_t e = hipGetLastError();
@@ -80,6 +91,28 @@ int64_t mf_stage_bytes(int wkind, int64_t M, int64_t K, int split, int wr = 1) {
   const int64_t rows = M < 8 * mf_blocks(M) ? M : 8 * mf_blocks(M);
   const int64_t bytes = rows * per * seg * 2;
   return bytes <= (wr > 1 ? kMaxStageBytesRows : kMaxStageBytes) ? bytes : -1;
+}
+
+// Segments of every wave when the split ranges and the waves divide the segments evenly into a count that a straight-line
+// kernel exists for (4, 8 or 16; with row groups 4 or 8), else 0.
+int mf_nseg_wave(int64_t nseg, int waves, int split, int xstage, int wr) {
+  if ((xstage & BP_XS_GENERAL) != 0 || nseg % split != 0 || (nseg / split) % waves != 0) return 0;
+  const int64_t n = nseg / split / waves;
+  return n == 4 || n == 8 || (n == 16 && wr == 1) ? static_cast<int>(n) : 0;
+}
+
+// Whether a vector launch without a prologue takes the kernel of skinny_wide.h (the same sums, bit for bit). Measured
+// both ways on one MI355X (us, this kernel / the wide one):
+//   - past 10 rows always (16 rows: 2048 x 2048 bf16 5.4 / 5.3, 8192 x 2048 10.3 / 9.6; int8 100352 x 2048 57 / 43);
+//   - at 9 and 10 rows, not where the straight-line kernels keep more CUs at work (8-row workgroups: 2048 x 2048 at 9
+//     rows bf16 5.0 / 5.3, int8 4.5 / 5.1; 2048 x 8192 bf16 12.1 / 12.6, int8, 8 segments a wave, 9.2 / 8.8) or share
+//     staged rows between row groups in bf16 (16384 x 2048 15.9 / 16.5; int8 11.8 / 9.3);
+//   - up to 8 rows never (8 rows: 16000 x 1984 bf16 12.7 / 13.1, 1152 x 1152 3.6 / 4.4).
+bool mf_wide_takes(int wkind, int64_t M, int64_t N, int split, int nseg_wave, int wr) {
+  if (M <= 8) return false;
+  if (M > 10 || nseg_wave == 0) return true;
+  if (N * split < 4096) return wkind == kInt8 && nseg_wave > 4;
+  return !(wkind == kBf16 && wr > 1);
 }
 
 constexpr int64_t kMaxVecK = int64_t{1} << 24;  // 2 x 64 rows x K bytes of activations < 2^31
@@ -163,21 +196,14 @@ int mf_launch(int wkind, const void* x, const void* w, const void* scale, int sc
 #ifdef BP_TIMELINE
   pro.tl = mf_timeline_buffer();
 #endif
-  // every wave has the same segment count when the split ranges and the waves divide the segments evenly
-  int nseg_wave = !general && nseg % split == 0 && (nseg / split) % waves == 0
-                      ? static_cast<int>(nseg / split / waves)
-                      : 0;
-  if (wr > 1 && nseg_wave == 16) nseg_wave = 0;  // the row-group kernels run the general loop there
-  MfFn fn = mf_pick(wkind, mf_blocks(M), rb, waves, vec, mode == 2 ? 1 : 0, xstage != 0, pro.kind != 0, nseg_wave,
-                    wr);
-  if (fn == nullptr && wr == 4) {
-    // row groups are a plan, not a K order: without a compiled kernel of 4 groups, 2 (the same LDS)
-    wr = 2;
-    fn = mf_pick(wkind, mf_blocks(M), rb, waves, vec, mode == 2 ? 1 : 0, xstage != 0, pro.kind != 0, nseg_wave, wr);
-  }
-  if (fn == nullptr && wr > 1 && pro.kind == 0) {
-    // without a row-group kernel (rows outside 9..16, rb or waves outside its menu), the same sums from one group,
-    // staged where the rows fit in the plain limit
+  const int nseg_wave = mf_nseg_wave(nseg, waves, split, general ? BP_XS_GENERAL : 0, wr);
+  const auto menu = [&](int groups) {
+    return vec ? mf_menu(wkind, mf_blocks(M), rb, waves, xstage != 0, groups) && !(pro.kind != 0 && groups != 1) : true;
+  };
+  if (!menu(wr) && wr == 4) wr = 2;  // row groups are a plan, not a K order: without 4 groups, 2 (the same LDS)
+  if (!menu(wr) && wr > 1 && pro.kind == 0) {
+    // without row groups (rows outside 9..16, rb or waves outside their menu), the same sums from one group, staged
+    // where the rows fit in the plain limit
     wr = 1;
     if (xstage) {
       lds = mf_stage_bytes(wkind, M, K, split, 1);
@@ -186,11 +212,25 @@ int mf_launch(int wkind, const void* x, const void* w, const void* scale, int sc
         lds = 0;
       }
     }
-    fn = mf_pick(wkind, mf_blocks(M), rb, waves, vec, mode == 2 ? 1 : 0, xstage != 0, false, nseg_wave);
   }
-  if (fn == nullptr) return BP_E_UNSUPPORTED;
+  if (!menu(wr)) return BP_E_UNSUPPORTED;
   if (split > 1 && (ws == nullptr || ws_bytes < static_cast<size_t>(split) * M * N * sizeof(float)))
     return BP_E_WORKSPACE;
+  if (vec && pro.kind == 0 && mf_wide_takes(wkind, M, N, split, nseg_wave, wr)) {
+    const MfWideTile t = mf_wide_tile(wkind, M, N, split);
+    if (t.wgs > 0x7fffffff) return BP_E_INVALID_ARG;
+    const MfWideFn wide = mf_wide_pick(wkind, t.mb, t.rp, waves, mode == 2 ? 1 : 0);
+    wide<<<dim3(static_cast<unsigned>(t.wgs), static_cast<unsigned>(split)), waves * kWave, 0, st>>>(
+        static_cast<const uint16_t*>(x), static_cast<const uint8_t*>(w), scale, scale_dt, static_cast<uint16_t*>(y),
+        static_cast<float*>(ws), static_cast<int>(M), N, K, split);
+    const int rc = mf_status();
+    if (rc != BP_OK || split == 1 || mode == 1) return rc;
+    return splitk_reduce_launch(static_cast<const float*>(ws), static_cast<uint16_t*>(y),
+                                wkind == kInt8 ? scale : nullptr, scale_dt, M, N, split, st);
+  }
+  const MfFn fn = mf_pick(wkind, mf_blocks(M), rb, waves, vec, mode == 2 ? 1 : 0, xstage != 0, pro.kind != 0, nseg_wave,
+                          wr);
+  if (fn == nullptr) return BP_E_UNSUPPORTED;
   const int64_t tiles = (N + 8 * rb * wr - 1) / (8 * rb * wr);
   if (tiles > 0x7fffffff) return BP_E_INVALID_ARG;
   fn<<<dim3(static_cast<unsigned>(tiles), static_cast<unsigned>(split)), waves * wr * kWave, static_cast<size_t>(lds),
@@ -262,11 +302,18 @@ int bp_skinny_mf_static(int wkind, const void* x, const void* w, const void* sca
 int bp_skinny_mf_supported(int wkind, int M, int rb, int waves, int xstage) {
   if (M < 1 || M > 64) return 0;
   const int wr = bp::mf_row_groups(xstage);
-  // the row-group kernels exist for the straight-line counts 4 and 8 and the general loop; report the general one
-  return bp::mf_pick(wkind, bp::mf_blocks(M), rb, waves, true, 0, (xstage & BP_XS_STAGE) != 0, false, 0, wr) !=
-                 nullptr
-             ? 1
-             : 0;
+  return bp::mf_menu(wkind, bp::mf_blocks(M), rb, waves, (xstage & BP_XS_STAGE) != 0, wr) ? 1 : 0;
+}
+
+int bp_skinny_mf_wide(int wkind, int64_t M, int64_t N, int64_t K, int waves, int split, int xstage) {
+  if ((wkind != bp::kBf16 && wkind != bp::kInt8) || M < 1 || M > 64 || N < 1 || K < 1 || waves < 1 || split < 1) return 0;
+  const int64_t seg = wkind == bp::kBf16 ? 64 : 128, nseg = K / seg;
+  if (K % seg != 0 || K >= bp::kMaxVecK) return 0;
+  if (split > nseg) split = static_cast<int>(nseg);
+  const int wr = bp::mf_row_groups(xstage);
+  if (!bp::mf_wide_takes(wkind, M, N, split, bp::mf_nseg_wave(nseg, waves, split, xstage, wr), wr)) return 0;
+  const bp::MfWideTile t = bp::mf_wide_tile(wkind, M, N, split);
+  return 256 * t.rp + t.mb;
 }
 
 int bp_skinny_mf_k_segment(int wkind) { return wkind == bp::kBf16 ? 64 : wkind == bp::kInt8 ? 128 : 0; }

@@ -422,9 +422,9 @@ __global__ __launch_bounds__(WAVES * WR * kWave) void skinny_mf_kernel(const uin
 }
 
 
-// Compiled menu: activation blocks MB in {1, 2, 4, 8} (M <= 8, 16, 32, 64) x row blocks RB in {1, 2, 4} (RB 4 up
-// to MB 2) x waves in {1, 2, 4, 8}; the SiLU epilogue and the LDS-staged activations up to MB 2; the element-load
-// variant at RB 1, 4 waves.
+// Compiled here (skinny_wide.hip holds the launches of more rows): activation blocks MB 1 and 2 (M <= 8, 16; MB 2 without
+// a prologue only straight-line) x row blocks RB in {1, 2, 4} x waves in {1, 2, 4, 8}; the element-load variant at MB 1,
+// 2, 4, 8, RB 1, 4 waves.
 template <int NSEG, int KIND, int MB, int RB, int EPI, bool XL, bool PRO>
 MfFn pick_waves(int waves) {
   switch (waves) {
@@ -441,9 +441,7 @@ MfFn pick_rb(int rb, int waves) {
   switch (rb) {
     case 1: return pick_waves<NSEG, KIND, MB, 1, EPI, XL, PRO>(waves);
     case 2: return pick_waves<NSEG, KIND, MB, 2, EPI, XL, PRO>(waves);
-    case 4:
-      if constexpr (MB <= 2) return pick_waves<NSEG, KIND, MB, 4, EPI, XL, PRO>(waves);
-      return nullptr;
+    case 4: return pick_waves<NSEG, KIND, MB, 4, EPI, XL, PRO>(waves);
     default: return nullptr;
   }
 }
@@ -465,12 +463,8 @@ MfFn pick_mb(int mb, int rb, int waves, bool vec) {
   }
   switch (mb) {
     case 1: return pick_rb<NSEG, KIND, 1, EPI, XL>(rb, waves);
-    case 2: return pick_rb<NSEG, KIND, 2, EPI, XL>(rb, waves);
-    case 4:
-      if constexpr (EPI == 0 && !XL) return pick_rb<NSEG, KIND, 4, EPI, XL>(rb, waves);
-      return nullptr;
-    case 8:
-      if constexpr (EPI == 0 && !XL) return pick_rb<NSEG, KIND, 8, EPI, XL>(rb, waves);
+    case 2:
+      if constexpr (NSEG > 0) return pick_rb<NSEG, KIND, 2, EPI, XL>(rb, waves);
       return nullptr;
     default: return nullptr;
   }
@@ -513,8 +507,8 @@ template <int NSEG, int KIND>
 MfFn mf_pick_kind(int mb, int rb, int waves, bool vec, int epi, bool xl, bool pro, int wr) {
   if (NSEG > 0 && !vec) return nullptr;
   if (wr != 1) {
-    if constexpr (NSEG == 16) {
-      return nullptr;  // K ranges of 16 segments a wave do not stage at 16 rows
+    if constexpr (NSEG == 0 || NSEG == 16) {
+      return nullptr;  // K ranges of 16 segments a wave do not stage at 16 rows; other counts run skinny_wide.hip
     } else {
       if (!vec || !xl || pro || mb != 2 || (wr != 2 && wr != 4)) return nullptr;
       if (epi == 0) return wr == 2 ? pick_wr_rb<NSEG, KIND, 0, 2>(rb, waves) : pick_wr_rb<NSEG, KIND, 0, 4>(rb, waves);

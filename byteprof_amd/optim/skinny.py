@@ -5,8 +5,8 @@ Drop-in for byteprof/optim/skinny.py: same names (`skinny_mm`, `get_cfg`, `_bm`,
 bf16 activations, fp32 accumulation, bf16 output; weights bf16 [N, K], int8 [N, K] with one scale per output row
 (bf16, fp16 or fp32), or int4 group-128 in the reference's tile-major format.
 
-bf16 and int8 run on one matrix-core kernel family for every row count (csrc/skinny_mf.h): one launch takes up to
-MAX_M = 64 activation rows and streams every weight byte once; the K order of every sum depends only on the shape's
+bf16 and int8 run on one matrix-core kernel family for every row count (csrc/skinny_mf.h, csrc/skinny_wide.h past 8 rows):
+one launch takes up to MAX_M = 64 activation rows and streams every weight byte once; the K order of every sum depends only on the shape's
 (waves, split), never on M, so output row i is bitwise the same whether it is computed alone or with up to 63 other
 rows (the reference's row-independence contract, test_skinny.py:110-120, here over M = 1..64). int4 runs on
 skinny_int4.hip (VALU dot products whose order also ignores M).
@@ -161,13 +161,14 @@ def segments_per_wave(kind: str, k: int, waves: int, split: int, xs: int = 0) ->
 def kernel_name(kind: str, n: int, k: int, m: int, cfg=None) -> str:
     """Name of the kernel instantiation a skinny_mm launch of m rows runs, as the profiler reports it (template
     arguments: kind, activation blocks, weight blocks, waves, vector loads, epilogue, staged activations, prologue,
-    segments per wave, row groups)."""
+    segments per wave, row groups; the wide kernel: kind, activation blocks, weight blocks, waves, epilogue)."""
     rb, waves, split, xs = _resolve(kind, n, k, m, cfg)
-    mb = 1 if m <= 8 else 2 if m <= 16 else 4 if m <= 32 else 8
+    wide = int(_lib.lib().bp_skinny_mf_wide(_KIND_CODE[kind], m, n, k, waves, split, xs))
+    if wide:
+        return f"skinny_wide_kernel<{_KIND_CODE[kind]}, {wide % 256}, {wide // 256}, {waves}, 0>"
+    mb = 1 if m <= 8 else 2
     wr = 4 if xs & XS_ROWS4 else 2 if xs & XS_ROWS2 else 1
     nseg = segments_per_wave(kind, k, waves, split, xs)
-    if wr > 1 and nseg == 16:
-        nseg = 0  # the row-group kernels run the general loop there
     return (f"skinny_mf_kernel<{_KIND_CODE[kind]}, {mb}, {rb}, {waves}, true, 0, "
             f"{'true' if xs & XS_STAGE else 'false'}, false, {nseg}, {wr}>")
 

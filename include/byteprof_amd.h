@@ -53,8 +53,9 @@ size_t bp_skinny_workspace_bytes(int64_t M, int64_t N, int split);
  *   BP_DT_BF16 / F16 / F32 on the fp32 sum), 1 <= M <= 64 per call (M = 0 or N = 0: no-op; K = 0: zeros).
  * One load instruction reads a 128-byte segment of 8 consecutive weight rows (one full line per row); the
  * activations are the MFMA's B operand (8 activation rows per 16 columns, the other 8 columns carry the other half of
- * the segment's K slots). Tile configuration: rb = 8-row weight blocks per workgroup (1, 2, 4; 4 up to M = 16),
- * waves = wavefronts sharing the workgroup's K segments (1, 2, 4, 8; segment s to wave s % waves), split = K ranges
+ * the segment's K slots); past 8..10 rows a kernel with 16 x 16 blocks takes over (bp_skinny_mf_wide), which picks its
+ * own tile and ignores rb and xstage. Tile configuration: rb = 8-row weight blocks per workgroup (1, 2, 4; 4 up to
+ * M = 16), waves = wavefronts sharing the workgroup's K segments (1, 2, 4, 8; segment s to wave s % waves), split = K ranges
  * in separate workgroups whose fp32 partials are added in split order by a second kernel (workspace as for
  * bp_skinny_workspace_bytes), xstage: flags BP_XS_STAGE (each workgroup copies its activation rows and K range to
  * LDS first; up to M = 16 and bp_skinny_mf_stage_bytes() >= 0; else the activation operands are loaded with the
@@ -77,6 +78,10 @@ size_t bp_skinny_workspace_bytes(int64_t M, int64_t N, int split);
 #define BP_XS_ROWS4 8
 int bp_skinny_mf_supported(int wkind, int M, int rb, int waves, int xstage);
 int bp_skinny_mf_k_segment(int wkind);
+/* Which kernel a bp_skinny_mf launch with vector loads runs: 0 the one of 8-row blocks, else 256 rp + mb: the wide kernel
+ * (9..64 rows) with rp 16-row weight blocks per wave and mb 16-row activation blocks per workgroup. The sums are the
+ * same. No counterpart in the reference (for profiling by kernel name). */
+int bp_skinny_mf_wide(int wkind, int64_t M, int64_t N, int64_t K, int waves, int split, int xstage);
 /* LDS bytes a launch with BP_XS_STAGE uses, or -1 when its activations do not fit (then the flag must be off). */
 int64_t bp_skinny_mf_stage_bytes(int wkind, int64_t M, int64_t K, int split);
 /* The same for a launch with BP_XS_STAGE and the row-group flags of xstage (their larger LDS limit). No counterpart in
