@@ -72,26 +72,33 @@ def k_segment(kind: str) -> int:
     return 64 if kind == "bf16" else 128
 
 
-def _default_waves(kind: str, k: int) -> int:
+def _default_waves(kind: str, n: int, k: int) -> int:
+    """Waves sharing K: 4 from 2 segments a wave on (1280 x 4736 bf16 at one row: 5.1 us with 4, 5.7 with 8); 8 for
+    int8 weights of few rows and a long K, whose 9..64-row launches have too few waves otherwise (1280 x 4736 at 16
+    rows: 7.4 us with 8, 8.7 with 4; at one row 4.8 and 4.6)."""
     nseg = -(-k // k_segment(kind))
-    waves = 1
-    while waves * 2 <= 8 and nseg // (waves * 2) >= 4:  # at least 4 segments per wave
-        waves *= 2
-    return waves
+    if kind == "int8" and nseg >= 32 and n < 4096:
+        return 8
+    return 4 if nseg >= 8 else 2 if nseg >= 4 else 1
 
 
-def _default_rb(n: int, bucket: int) -> int:
-    blocks = -(-n // 8)
-    if bucket > 16:
+def _default_rb(kind: str, n: int, bucket: int) -> int:
+    """8-row weight blocks per workgroup: 1 while that leaves no more than two workgroups per CU, else 4 (each
+    activation operand then serves 32 weight rows: 5000 x 6016 bf16 at 8 rows 21.5 us with 1, 16.8 with 4; int8 at one
+    row 10.1 and 9.2), but 1 for bf16 at one row (16000 x 1984: 12.0 us with 1, 12.3 with 4). Past 8 rows the launch
+    picks its own tile."""
+    if n < 4096 or bucket > 8 or (kind == "bf16" and bucket == 1):
         return 1
-    return 2 if blocks >= 2048 else 1
+    return 4
 
 
 def _default_split(kind: str, n: int, k: int, waves: int) -> int:
+    """K ranges in separate workgroups: only for a K so long that a wave's share outweighs the reduce launch (about
+    2.5 us: 1920 x 7168 bf16 at one row takes 6.8 us without a split, 9.1 with 2; 300 x 1024 2.6 and 4.4)."""
     blocks = -(-n // 8)
     nseg = -(-k // k_segment(kind))
     split = 1
-    while blocks * split < 256 and nseg // (waves * split * 2) >= 2:
+    while blocks * split < 256 and nseg // (waves * split * 2) >= 64:
         split *= 2
     return split
 
@@ -109,13 +116,13 @@ def _table_plan(kind: str, n: int, k: int, m: int, pro: bool = False) -> tuple[i
     bucket = _bucket(m)
     entry = _TABLE.get((kind, n, k))
     if entry is not None:
-        rb = int(entry.get("rb", {}).get(str(bucket), _default_rb(n, bucket)))
+        rb = int(entry.get("rb", {}).get(str(bucket), _default_rb(kind, n, bucket)))
         if pro:
             rb = int(entry.get("rb_pro", {}).get(str(bucket), rb))
         xs = int(entry.get("xs", {}).get(str(bucket), 0))
         return rb, int(entry["waves"]), int(entry.get("split", 1)), xs
-    waves = _default_waves(kind, k)
-    return _default_rb(n, bucket), waves, _default_split(kind, n, k, waves), int(n >= 16384)
+    waves = _default_waves(kind, n, k)
+    return _default_rb(kind, n, bucket), waves, _default_split(kind, n, k, waves), 0
 
 
 def _resolve(kind: str, n: int, k: int, m: int, cfg, pro: bool = False) -> tuple[int, int, int, int]:
