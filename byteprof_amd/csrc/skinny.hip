@@ -4,8 +4,11 @@
 //
 // Reference semantics: byteprof/optim/skinny.py:84-90 (_split_reduce).
 
+#include <algorithm>
+
 #include "byteprof_amd.h"
 #include "common.h"
+#include "skinny_int4.h"
 #include "skinny_mf_kernel.h"  // MfPro
 
 namespace bp {
@@ -62,8 +65,9 @@ constexpr int64_t kInt4ProMaxRows = 8;
 // (split 1, the matrix-core kernel, bf16 scales, M <= 8 and (2 M + 2) K x 2 bytes <= 64 KiB), as bp_skinny_mf_pro's.
 int skinny_int4_launch(const void* x, const void* packed, const void* scale, int scale_dt, const void* zero, void* y,
                        int64_t M, int64_t N, int64_t K, int tile_rows, int waves, int split, void* ws,
-                       size_t ws_bytes, void* stream, int epi = 0, const BpPrologue* prologue = nullptr) {
-  if (M < 0 || N < 0 || K < 0 || M > 16 || K % 128 != 0) return BP_E_INVALID_ARG;
+                       size_t ws_bytes, void* stream, int epi = 0, const BpPrologue* prologue = nullptr,
+                       int64_t max_rows = 16) {
+  if (M < 0 || N < 0 || K < 0 || M > max_rows || K % 128 != 0) return BP_E_INVALID_ARG;
   if (epi != 0 && (split != 1 || N % 2 != 0)) return BP_E_UNSUPPORTED;
   MfPro pro{0, 0.f, nullptr, nullptr, nullptr, 0, nullptr, nullptr};
   if (prologue != nullptr && prologue->kind != 0) {
@@ -106,17 +110,37 @@ int skinny_int4_launch(const void* x, const void* packed, const void* scale, int
   const bool mf = N % 4 == 0 && reinterpret_cast<uintptr_t>(zero) % 8 == 0 &&
                   reinterpret_cast<uintptr_t>(scale) % sc_align == 0 && K < (int64_t{1} << 24);
   if ((epi != 0 || pro.kind != 0) && !mf) return BP_E_UNSUPPORTED;
-  Int4MfFn mf_fn = mf ? int4_mf_pick(tile_rows, waves, scale_dt, epi, pro.kind != 0) : nullptr;
+  const int64_t tiles = tile_rows > 0 ? (N + tile_rows - 1) / tile_rows : 0;
+  if (tiles > 0x7fffffff) return BP_E_INVALID_ARG;
+  const int nb = mf && pro.kind == 0 ? int4_wide_nb(M, K, tiles) : 0;
+  if (nb == 0 && M > 16) {  // the VALU kernel: 16 rows a launch
+    for (int64_t r = 0; r < M; r += 16) {
+      const int rc = skinny_int4_launch(static_cast<const uint16_t*>(x) + r * K, packed, scale, scale_dt, zero,
+                                        static_cast<uint16_t*>(y) + r * N, std::min<int64_t>(16, M - r), N, K, tile_rows,
+                                        waves, split, ws, ws_bytes, stream, epi);
+      if (rc != BP_OK) return rc;
+    }
+    return BP_OK;
+  }
+  const Int4WideFn wide = nb > 0 ? int4_wide_pick(nb, tile_rows, waves, scale_dt, epi) : nullptr;
+  if (nb > 0 && wide == nullptr) return BP_E_UNSUPPORTED;
+  Int4MfFn mf_fn = mf && nb == 0 ? int4_mf_pick(tile_rows, waves, scale_dt, epi, pro.kind != 0) : nullptr;
   Int4Fn fn = mf ? nullptr : int4_pick(row_bucket(M), tile_rows, waves);
-  if (mf_fn == nullptr && fn == nullptr) return BP_E_UNSUPPORTED;
+  if (mf_fn == nullptr && fn == nullptr && wide == nullptr) return BP_E_UNSUPPORTED;
   const int64_t groups = K / 128;
   if (split > groups) split = static_cast<int>(groups);
   if (split > 1 && (ws == nullptr || ws_bytes < static_cast<size_t>(split) * M * N * sizeof(float)))
     return BP_E_WORKSPACE;
-  const int64_t tiles = (N + tile_rows - 1) / tile_rows;
-  if (tiles > 0x7fffffff) return BP_E_INVALID_ARG;
   dim3 grid(static_cast<unsigned>(tiles), static_cast<unsigned>(split));
-  if (mf_fn != nullptr) {
+  if (wide != nullptr) {
+    // every XCD's run of tiles (the longest), each with its activation tiles
+    const int64_t wgs = (tiles + kXcds - 1) / kXcds * kXcds * ((M + 16 * nb - 1) / (16 * nb));
+    if (wgs > 0x7fffffff) return BP_E_INVALID_ARG;
+    grid.x = static_cast<unsigned>(wgs);
+    wide<<<grid, waves * kWave, 0, st>>>(static_cast<const uint16_t*>(x), static_cast<const uint8_t*>(packed), scale,
+                                         static_cast<const uint16_t*>(zero), static_cast<uint16_t*>(y),
+                                         static_cast<float*>(ws), static_cast<int>(M), N, K, split);
+  } else if (mf_fn != nullptr) {
     const size_t lds = pro.kind != 0 ? static_cast<size_t>((2 * M + 2) * K * 2) : 0;
     mf_fn<<<grid, waves * kWave, lds, st>>>(static_cast<const uint16_t*>(x), static_cast<const uint8_t*>(packed),
                                             scale, scale_dt, static_cast<const uint16_t*>(zero),
@@ -155,6 +179,13 @@ int bp_skinny_int4(const void* x, const void* packed, const void* scale, int sca
                    size_t workspace_bytes, void* stream) {
   return bp::skinny_int4_launch(x, packed, scale, scale_dtype, zero, y, M, N, K, tile_rows, waves, split, workspace,
                                 workspace_bytes, stream);
+}
+
+int bp_skinny_int4_rows(const void* x, const void* packed, const void* scale, int scale_dtype, const void* zero, void* y,
+                        int64_t M, int64_t N, int64_t K, int tile_rows, int waves, int split, void* workspace,
+                        size_t workspace_bytes, void* stream) {
+  return bp::skinny_int4_launch(x, packed, scale, scale_dtype, zero, y, M, N, K, tile_rows, waves, split, workspace,
+                                workspace_bytes, stream, 0, nullptr, 64);
 }
 
 int bp_skinny_int4_pro(const void* x, const void* packed, const void* scale, int scale_dtype, const void* zero, void* y,

@@ -32,6 +32,7 @@
 
 #include "byteprof_amd.h"
 #include "common.h"
+#include "skinny_int4.h"
 #include "skinny_mf_kernel.h"  // MfPro and mf_prologue: the norm prologue the matrix-core kernels share
 
 namespace bp {
@@ -42,16 +43,6 @@ using Int4MfFn = void (*)(const uint16_t*, const uint8_t*, const void*, int, con
                           int64_t, int64_t, int, MfPro);
 
 namespace {
-
-constexpr uint32_t kBf16Exp128 = 0x43434343u;  // 0x43 in every byte: bf16 0x43xx = 128 + xx
-constexpr uint32_t kBf16OnePair = 0x3F803F80u; // two bf16 1.0
-
-// Four codes (bytes of m, each below 128) as two bf16 pairs (128 + byte).
-__device__ __forceinline__ void codes_to_bf16(uint32_t m, uint32_t& p01, uint32_t& p23) {
-  // v_perm_b32 (S0 = m: bytes 4..7, S1 = 0x43434343: bytes 0..3): result bytes [m0, 0x43, m1, 0x43] / [m2, .., m3, ..]
-  p01 = __builtin_amdgcn_perm(m, kBf16Exp128, 0x00050004u);
-  p23 = __builtin_amdgcn_perm(m, kBf16Exp128, 0x00070006u);
-}
 
 template <int MT, int RB, int WAVES>
 __global__ __launch_bounds__(WAVES * kWave) void skinny_int4_kernel(const uint16_t* __restrict__ x,
@@ -189,12 +180,6 @@ struct I4Slot {
   u32x4 xv[4];       // activations at K 16 kb + 0..7, + 8..15, 64 + 16 kb + 0..7, + 8..15 of the lane's column
   uint32_t rv[NR];   // dwords 64 c + l of the group's record
 };
-
-__device__ __forceinline__ float half_bits_to_float(uint32_t h) {
-  return static_cast<float>(__builtin_bit_cast(_Float16, static_cast<uint16_t>(h)));
-}
-
-using u32x2 = unsigned __attribute__((ext_vector_type(2)));
 
 // PRO (up to 8 activation rows, split 1): the rows staged in LDS with gamma, the residual rows and gamma2 (dynamic
 // shared memory, (2 M + 2) K bf16), transformed by mf_prologue (the norm kernel's arithmetic: the product equals a norm launch

@@ -9,7 +9,7 @@ bf16 and int8 run on one matrix-core kernel family for every row count (csrc/ski
 one launch takes up to MAX_M = 64 activation rows and streams every weight byte once; the K order of every sum depends only on the shape's
 (waves, split), never on M, so output row i is bitwise the same whether it is computed alone or with up to 63 other
 rows (the reference's row-independence contract, test_skinny.py:110-120, here over M = 1..64). int4 runs on
-skinny_int4.hip (VALU dot products whose order also ignores M).
+skinny_int4.hip and skinny_int4_wide.hip (their order ignores M too).
 
 `cfg` is (rows, waves, split) for the bf16 / int8 kernel (rows: weight rows per workgroup, a multiple of 8;
 waves: wavefronts sharing a workgroup's K range; split: K ranges in separate workgroups, added in fixed order) or
@@ -339,7 +339,7 @@ def skinny_mm(x: torch.Tensor, w: torch.Tensor, scale: torch.Tensor | None = Non
     return y
 
 
-INT4_ROWS_PER_LAUNCH = 16  # activation rows per launch of the int4 kernel
+INT4_ROWS_PER_LAUNCH = MAX_M  # activation rows per launch of the int4 kernel
 
 
 INT4_TILES = (16, 32, 64)  # tile rows of the int4 matrix-core kernel on gfx950
@@ -400,10 +400,10 @@ def _launch_int4(x: torch.Tensor, w: torch.Tensor, scale: torch.Tensor, zero: to
     if split > 1:
         ws_bytes = L.bp_skinny_workspace_bytes(m, n, split)
         ws = torch.empty(ws_bytes // 4, dtype=torch.float32, device=x.device)
-    rc = L.bp_skinny_int4(x.data_ptr(), w.data_ptr(), scale.data_ptr(), _lib.TORCH_DT[scale.dtype], zero.data_ptr(),
-                          y.data_ptr(), m, n, k, tile_rows, waves, split, _lib.ptr(ws), ws_bytes,
-                          _lib.stream_ptr(x.device))
-    _lib.check(rc, "bp_skinny_int4")
+    rc = L.bp_skinny_int4_rows(x.data_ptr(), w.data_ptr(), scale.data_ptr(), _lib.TORCH_DT[scale.dtype], zero.data_ptr(),
+                               y.data_ptr(), m, n, k, tile_rows, waves, split, _lib.ptr(ws), ws_bytes,
+                               _lib.stream_ptr(x.device))
+    _lib.check(rc, "bp_skinny_int4_rows")
 
 
 def quantize_int4(w: torch.Tensor, tile_rows: int = 32) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor]:

@@ -214,6 +214,12 @@ int bp_skinny_int4_config_supported(int mt, int tile_rows, int waves);
 int bp_skinny_int4(const void* x, const void* packed, const void* scale, int scale_dtype, const void* zero, void* y,
                    int64_t M, int64_t N, int64_t K, int tile_rows, int waves, int split, void* workspace,
                    size_t workspace_bytes, void* stream);
+/* bp_skinny_int4 for 1 <= M <= 64 rows: one launch (skinny_int4_wide.hip) where the matrix-core kernel applies, else one
+ * per 16 rows; the same bits as bp_skinny_int4 on each row. Replaces: byteprof/optim/skinny.py:111-133 (_launch) for the
+ * row buckets 32 and 64 with MODE 3 weights. */
+int bp_skinny_int4_rows(const void* x, const void* packed, const void* scale, int scale_dtype, const void* zero, void* y,
+                        int64_t M, int64_t N, int64_t K, int tile_rows, int waves, int split, void* workspace,
+                        size_t workspace_bytes, void* stream);
 /* bp_skinny_int4 of an interleaved gate|up weight ([2 ffn, K] packed: row 2f the gate row f, row 2f + 1 the up row
  * f) with the SiLU product as the epilogue: out [M, ffn] = bf16(bf16(silu(bf16(g))) * bf16(u)), equal bit for bit to
  * bp_skinny_int4 (same tile rows and waves, split 1) followed by bp_decode_silu_mul_rows (interleaved). The

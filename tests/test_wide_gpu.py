@@ -1,4 +1,4 @@
-"""The wide matrix-core kernel (9..64 activation rows): every output row equal bit for bit to the same row computed alone
+"""The wide matrix-core kernels (bf16 / int8: 9..64 activation rows; int4: 1..64): every output row equal bit for bit to the same row computed alone
 by the one-row kernel at the same K order, and to the oracle, at the edges of its tiles: a single weight row, partial
 blocks of 16 weight rows, partial activation blocks, activation tiles in separate workgroups, waves without a segment,
 split K, the SiLU epilogue's odd last pair, unaligned output rows."""
@@ -78,3 +78,26 @@ def test_the_rule_takes_every_tile_it_may_pick():
                     code = L.bp_skinny_mf_wide(kind, m, n, 32 * seg, waves, 1, 0)
                     assert (code == 0) if m <= 8 else (code // 256 in (0, 1, 2, 4) and code % 256 <= 4)
                     assert m <= 10 or code > 0
+
+
+@pytest.mark.parametrize("tile_rows", [16, 32, 64])
+@pytest.mark.parametrize("n,groups,waves,split,sdt", [(4, 1, 4, 1, None), (68, 3, 2, 1, torch.float16),
+                                                      (300, 9, 8, 2, torch.float32), (1000, 32, 1, 1, None),
+                                                      (17000, 2, 4, 1, None)])
+def test_int4_rows_equal_the_one_row_launch(tile_rows, n, groups, waves, split, sdt):
+    """bp_skinny_int4_rows at 1..64 rows (one and two activation blocks per workgroup, one and several activation tiles,
+    partial weight tiles, waves without a group): each row equal bit for bit to its own launch, which with these few tiles
+    is the 16-row kernel's (17000 rows: the wide one's)."""
+    k = groups * S.GROUP
+    w = (torch.randn(n, k, generator=torch.Generator(device=DEV).manual_seed(n), device=DEV) * 0.02).to(torch.bfloat16)
+    packed, scale, zero = S.quantize_int4(w, tile_rows)
+    scale = scale if sdt is None else scale.to(sdt)
+    x = randn_x(64, k, seed=n)
+    ones = torch.cat([S.skinny_mm(x[r:r + 1].contiguous(), packed, scale, zero, cfg=(waves, split)) for r in range(64)])
+    for m in (5, 9, 16, 17, 32, 33, 49, 64):
+        got = S.skinny_mm(x[:m].contiguous(), packed, scale, zero, cfg=(waves, split))
+        assert torch.equal(got.view(torch.int16), ones[:m].view(torch.int16)), m
+    check_against_oracle(got, x, S.dequantize("int4", packed, scale, zero).cpu().numpy())
+    assert _lib.lib().bp_skinny_int4_rows(x.data_ptr(), packed.data_ptr(), scale.data_ptr(), _lib.TORCH_DT[scale.dtype],
+                                          zero.data_ptr(), got.data_ptr(), 65, n, k, tile_rows, waves, 1, None, 0,
+                                          _lib.stream_ptr(DEV)) == _lib.BP_E_INVALID_ARG
