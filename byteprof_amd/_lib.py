@@ -56,8 +56,10 @@ SIGNATURES: dict[str, tuple] = {
     "bp_skinny_int4_config_supported": (_c_int, [_c_int, _c_int, _c_int]),
     "bp_skinny_int4": (_c_int, [_c_vp, _c_vp, _c_vp, _c_int, _c_vp, _c_vp, _c_i64, _c_i64, _c_i64, _c_int, _c_int,
                                 _c_int, _c_vp, _c_size, _c_vp]),
+    "bp_skinny_mf_rows": (_c_int, [_c_int, _c_vp, _c_vp, _c_vp, _c_int, _c_vp, _c_i64, _c_i64, _c_i64, _c_int, _c_int,
+                                   _c_int, _c_vp, _c_size, _c_vp]),
     "bp_skinny_int4_rows": (_c_int, [_c_vp, _c_vp, _c_vp, _c_int, _c_vp, _c_vp, _c_i64, _c_i64, _c_i64, _c_int, _c_int,
-                                     _c_int, _c_vp, _c_size, _c_vp]),
+                                     _c_int, _c_int, _c_vp, _c_size, _c_vp]),
     "bp_skinny_int4_silu": (_c_int, [_c_vp, _c_vp, _c_vp, _c_int, _c_vp, _c_vp, _c_i64, _c_i64, _c_i64, _c_int,
                                      _c_int, _c_vp]),
     "bp_skinny_int4_pro": (_c_int, [_c_vp, _c_vp, _c_vp, _c_int, _c_vp, _c_vp, _c_i64, _c_i64, _c_i64, _c_int,

@@ -116,7 +116,7 @@ int skinny_int4_launch(const void* x, const void* packed, const void* scale, int
   if (nb == 0 && M > 16) {  // the VALU kernel: 16 rows a launch
     for (int64_t r = 0; r < M; r += 16) {
       const int rc = skinny_int4_launch(static_cast<const uint16_t*>(x) + r * K, packed, scale, scale_dt, zero,
-                                        static_cast<uint16_t*>(y) + r * N, std::min<int64_t>(16, M - r), N, K, tile_rows,
+                                        static_cast<uint16_t*>(y) + r * (epi != 0 ? N / 2 : N), std::min<int64_t>(16, M - r), N, K, tile_rows,
                                         waves, split, ws, ws_bytes, stream, epi);
       if (rc != BP_OK) return rc;
     }
@@ -182,10 +182,11 @@ int bp_skinny_int4(const void* x, const void* packed, const void* scale, int sca
 }
 
 int bp_skinny_int4_rows(const void* x, const void* packed, const void* scale, int scale_dtype, const void* zero, void* y,
-                        int64_t M, int64_t N, int64_t K, int tile_rows, int waves, int split, void* workspace,
-                        size_t workspace_bytes, void* stream) {
-  return bp::skinny_int4_launch(x, packed, scale, scale_dtype, zero, y, M, N, K, tile_rows, waves, split, workspace,
-                                workspace_bytes, stream, 0, nullptr, 64);
+                        int64_t M, int64_t N, int64_t K, int tile_rows, int waves, int split, int epilogue,
+                        void* workspace, size_t workspace_bytes, void* stream) {
+  if (epilogue < 0 || epilogue > 1) return BP_E_INVALID_ARG;
+  return bp::skinny_int4_launch(x, packed, scale, scale_dtype, zero, y, M, epilogue && N >= 0 ? 2 * N : N, K, tile_rows,
+                                waves, split, workspace, workspace_bytes, stream, epilogue, nullptr, 0x7fffff00);
 }
 
 int bp_skinny_int4_pro(const void* x, const void* packed, const void* scale, int scale_dtype, const void* zero, void* y,

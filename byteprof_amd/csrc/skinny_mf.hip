@@ -117,6 +117,22 @@ bool mf_wide_takes(int wkind, int64_t M, int64_t N, int split, int nseg_wave, in
 
 constexpr int64_t kMaxVecK = int64_t{1} << 24;  // 2 x 64 rows x K bytes of activations < 2^31
 
+// A launch of the wide kernel (vector operands, any M >= 1); mode as mf_launch's.
+int mf_wide_launch(int wkind, const void* x, const void* w, const void* scale, int scale_dt, void* y, int64_t M,
+                   int64_t N, int64_t K, int waves, int split, void* ws, hipStream_t st, int mode) {
+  const MfWideTile t = mf_wide_tile(wkind, M, N, split);
+  if (t.wgs > 0x7fffffff || M > 0x7fffff00) return BP_E_INVALID_ARG;
+  const MfWideFn fn = mf_wide_pick(wkind, t.mb, t.rp, waves, mode == 2 ? 1 : 0);
+  if (fn == nullptr) return BP_E_UNSUPPORTED;
+  fn<<<dim3(static_cast<unsigned>(t.wgs), static_cast<unsigned>(split)), waves * kWave, 0, st>>>(
+      static_cast<const uint16_t*>(x), static_cast<const uint8_t*>(w), scale, scale_dt, static_cast<uint16_t*>(y),
+      static_cast<float*>(ws), static_cast<int>(M), N, K, split);
+  const int rc = mf_status();
+  if (rc != BP_OK || split == 1 || mode == 1) return rc;
+  return splitk_reduce_launch(static_cast<const float*>(ws), static_cast<uint16_t*>(y),
+                              wkind == kInt8 ? scale : nullptr, scale_dt, M, N, split, st);
+}
+
 // mode 0: y (split > 1: partials then the reduce); 1: partials only (split >= 2, y unused); 2: SiLU epilogue.
 int mf_launch(int wkind, const void* x, const void* w, const void* scale, int scale_dt, void* y, int64_t M,
               int64_t N, int64_t K, int rb, int waves, int split, int xstage, void* ws, size_t ws_bytes, void* stream,
@@ -216,18 +232,8 @@ int mf_launch(int wkind, const void* x, const void* w, const void* scale, int sc
   if (!menu(wr)) return BP_E_UNSUPPORTED;
   if (split > 1 && (ws == nullptr || ws_bytes < static_cast<size_t>(split) * M * N * sizeof(float)))
     return BP_E_WORKSPACE;
-  if (vec && pro.kind == 0 && mf_wide_takes(wkind, M, N, split, nseg_wave, wr)) {
-    const MfWideTile t = mf_wide_tile(wkind, M, N, split);
-    if (t.wgs > 0x7fffffff) return BP_E_INVALID_ARG;
-    const MfWideFn wide = mf_wide_pick(wkind, t.mb, t.rp, waves, mode == 2 ? 1 : 0);
-    wide<<<dim3(static_cast<unsigned>(t.wgs), static_cast<unsigned>(split)), waves * kWave, 0, st>>>(
-        static_cast<const uint16_t*>(x), static_cast<const uint8_t*>(w), scale, scale_dt, static_cast<uint16_t*>(y),
-        static_cast<float*>(ws), static_cast<int>(M), N, K, split);
-    const int rc = mf_status();
-    if (rc != BP_OK || split == 1 || mode == 1) return rc;
-    return splitk_reduce_launch(static_cast<const float*>(ws), static_cast<uint16_t*>(y),
-                                wkind == kInt8 ? scale : nullptr, scale_dt, M, N, split, st);
-  }
+  if (vec && pro.kind == 0 && mf_wide_takes(wkind, M, N, split, nseg_wave, wr))
+    return mf_wide_launch(wkind, x, w, scale, scale_dt, y, M, N, K, waves, split, ws, st, mode);
   const MfFn fn = mf_pick(wkind, mf_blocks(M), rb, waves, vec, mode == 2 ? 1 : 0, xstage != 0, pro.kind != 0, nseg_wave,
                           wr);
   if (fn == nullptr) return BP_E_UNSUPPORTED;
@@ -240,6 +246,38 @@ int mf_launch(int wkind, const void* x, const void* w, const void* scale, int sc
   if (rc != BP_OK || split == 1 || mode == 1) return rc;
   return splitk_reduce_launch(static_cast<const float*>(ws), static_cast<uint16_t*>(y),
                               wkind == kInt8 ? scale : nullptr, scale_dt, M, N, split, st);
+}
+
+// Any number of rows at the plan (waves, split): the wide kernel over all of them in one launch, a few rows (or operands
+// that the vector loads cannot take) through mf_launch. epi 1: the SiLU product of N / 2 interleaved pairs (split 1).
+int mf_rows_launch(int wkind, const void* x, const void* w, const void* scale, int scale_dt, void* y, int64_t M,
+                   int64_t N, int64_t K, int waves, int split, int epi, void* ws, size_t ws_bytes, void* stream) {
+  if ((wkind != kBf16 && wkind != kInt8) || (epi != 0 && epi != 1)) return BP_E_UNSUPPORTED;
+  if (M < 0 || N < 0 || K < 0) return BP_E_INVALID_ARG;
+  if (epi == 1 && (split != 1 || N % 2 != 0)) return BP_E_UNSUPPORTED;
+  const int64_t most = epi == 1 ? 16 : 64;  // rows of one mf_launch
+  const int64_t seg = wkind == kBf16 ? 64 : 128;
+  const bool vec = K > 0 && K % seg == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0 &&
+                   reinterpret_cast<uintptr_t>(w) % 16 == 0 && K < kMaxVecK;
+  if (M <= most || !vec) {
+    const int64_t step = M <= most ? std::max<int64_t>(M, 1) : most;
+    for (int64_t r = 0; r < std::max<int64_t>(M, 1); r += step) {
+      const int rc = mf_launch(wkind, static_cast<const uint16_t*>(x) + r * K, w, scale, scale_dt,
+                               static_cast<uint16_t*>(y) + r * (epi == 1 ? N / 2 : N), std::min(step, M - r), N, K, 1,
+                               waves, split, 0, ws, ws_bytes, stream, epi == 1 ? 2 : 0);
+      if (rc != BP_OK) return rc;
+    }
+    return BP_OK;
+  }
+  if (N == 0) return BP_OK;
+  if (x == nullptr || w == nullptr || y == nullptr) return BP_E_INVALID_ARG;
+  if (wkind == kInt8 && (scale == nullptr || scale_dt < BP_DT_BF16 || scale_dt > BP_DT_F32)) return BP_E_INVALID_ARG;
+  if (split < 1 || split > 1024 || !mf_menu(wkind, 1, 1, waves, false, 1)) return BP_E_UNSUPPORTED;
+  if (split > K / seg) split = static_cast<int>(K / seg);
+  if (split > 1 && (ws == nullptr || ws_bytes < static_cast<size_t>(split) * M * N * sizeof(float)))
+    return BP_E_WORKSPACE;
+  return mf_wide_launch(wkind, x, w, scale, scale_dt, y, M, N, K, waves, split, ws, static_cast<hipStream_t>(stream),
+                        epi == 1 ? 2 : 0);
 }
 
 // The split-K partials of bp_skinny_mf_static: a fixed device array instead of a caller's workspace. Each GPU the
@@ -333,6 +371,13 @@ int bp_skinny_mf(int wkind, const void* x, const void* w, const void* scale, int
                  size_t workspace_bytes, void* stream) {
   return bp::mf_launch(wkind, x, w, scale, scale_dtype, y, M, N, K, rb, waves, split, xstage, workspace,
                        workspace_bytes, stream, 0);
+}
+
+int bp_skinny_mf_rows(int wkind, const void* x, const void* w, const void* scale, int scale_dtype, void* y, int64_t M,
+                      int64_t N, int64_t K, int waves, int split, int epilogue, void* workspace, size_t workspace_bytes,
+                      void* stream) {
+  return bp::mf_rows_launch(wkind, x, w, scale, scale_dtype, y, M, epilogue == 1 && N >= 0 ? 2 * N : N, K, waves, split,
+                            epilogue, workspace, workspace_bytes, stream);
 }
 
 int bp_skinny_mf_partials(int wkind, const void* x, const void* w, int64_t M, int64_t N, int64_t K, int rb,

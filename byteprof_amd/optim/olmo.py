@@ -18,8 +18,9 @@ int4 (group-128 codes). The gate and up rows are interleaved (row 2n gate n, row
 computes the projection and the SiLU product (bp_skinny_mf_silu, bp_skinny_int4_silu). Every linear runs on a
 matrix-core kernel whose rows do not depend on how many rows share a launch: a verify pass of s rows computes each
 row exactly as the one-token step.
-The prompt is fed one position at a time through the same step (the reference prefills with one batched
-forward; the cache contents and the first new token are the same up to rounding).
+The prompt runs in passes of up to PREFILL_ROWS rows (the reference prefills with one batched forward): every row gets
+the bits that the one-token step at its position computes, so the caches, the logits and the first new token are those
+of feeding the positions one at a time.
 """
 
 from __future__ import annotations
@@ -35,6 +36,7 @@ from . import skinny as S
 
 MAX_CACHE_LEN = 1024  # the reference's static cache length (olmo.py:16)
 ROPE_ATTENTION_ROWS = 16  # most rows of one fused q/k-norm + RoPE + cache + attention launch
+PREFILL_ROWS = 256  # most prompt rows of one pass (its buffers: about 5 (H + F) KiB a row, allocated at the first prompt)
 VERIFY_ROWS = 16  # rows of the verify-pass buffers (allocated once per decoder, never reallocated)
 PRO_MAX_ROWS = {"bf16": 3, "int8": 1, "int4": 1}  # most rows of a linear launch with the norm as its prologue
 INT4_PRO_LDS_BYTES = 64 * 1024  # the int4 kernel's norm prologue: rows, gamma, residual rows, gamma2, (2 M + 2) K bf16
@@ -410,6 +412,108 @@ class OlmoDecoder:
         c(L.bp_draft_verify_next(self.v_ids.data_ptr(), self.v_tok.data_ptr(), self.v_out.data_ptr(),
                                  self.v_pos.data_ptr(), s, self.smax, st), "bp_draft_verify_next")
 
+    def _prefill_buffers(self) -> dict[str, torch.Tensor]:
+        """The buffers of prompt passes (allocated at the first prompt of more than one token and kept)."""
+        bufs = getattr(self, "_prefill", None)
+        if bufs is None:
+            H, F, n = self.cfg.hidden, self.cfg.ffn, PREFILL_ROWS
+            z = lambda *shape, dtype=torch.bfloat16: torch.empty(*shape, dtype=dtype, device=self.device)  # noqa: E731
+            bufs = {"ids": z(n, dtype=torch.int64), "x": z(n, H), "q": z(n, H), "attn": z(n, H), "o": z(n, H),
+                    "qkv": z(n, 3 * H), "act": z(n, F)}
+            plans = {(rows, k): self._plan(rows, k, 1)[1:3] for rows, k in ((3 * H, H), (H, H), (2 * F, H), (H, F))}
+            need = max((split * n * rows for (rows, _), (_, split) in plans.items() if split > 1), default=0)
+            if plans[(2 * F, H)][1] > 1:  # a split gate|up has no SiLU epilogue
+                bufs["gu"] = z(n, 2 * F)
+            bufs["ws"] = z(max(1, need), dtype=torch.float32)
+            self._prefill, self._prefill_plans = bufs, plans
+        return bufs
+
+    def _rows_mm(self, x: torch.Tensor, args: tuple, out: torch.Tensor, rows: int, n: int, k: int, st: int,
+                 silu: bool = False) -> None:
+        """out[:rows] = the n x k linear of x[:rows] (silu: the gate|up product), any number of rows in one call, at the
+        K order that the one-token step's launches of this shape use."""
+        L, ws = _lib.lib(), self._prefill["ws"]
+        waves, split = self._prefill_plans[(n, k)]
+        nout = n // 2 if silu else n
+        if self.kind == "int4":
+            packed, scale, zero = args
+            rc = L.bp_skinny_int4_rows(x.data_ptr(), packed.data_ptr(), scale.data_ptr(), _lib.TORCH_DT[scale.dtype],
+                                       zero.data_ptr(), out.data_ptr(), rows, nout, k, int(packed.shape[2]), waves, split,
+                                       int(silu), ws.data_ptr(), ws.numel() * 4, st)
+            _lib.check(rc, "bp_skinny_int4_rows")
+            return
+        sc, sdt = (args[1].data_ptr(), _lib.TORCH_DT[args[1].dtype]) if self.kind == "int8" else (None, 0)
+        rc = L.bp_skinny_mf_rows(S._KIND_CODE[self.kind], x.data_ptr(), args[0].data_ptr(), sc, sdt, out.data_ptr(), rows,
+                                 nout, k, waves, split, int(silu), ws.data_ptr(), ws.numel() * 4, st)
+        _lib.check(rc, "bp_skinny_mf_rows")
+
+    def prefill(self, ids: torch.Tensor) -> None:
+        """The prompt ids [L] at positions 0 .. L - 1: fills the caches, leaves the last position's logits in `logits`,
+        the first new token in tok and L in pos, bit for bit as L calls of step() from position 0 would. Passes of up to
+        PREFILL_ROWS rows: 160 positions of the OLMo-2-1B shape in one (9 launches a layer) instead of 160 steps of 83
+        launches. After the last layer's cache write only the prompt's last row goes on."""
+        length = ids.shape[0]
+        self.pos.zero_()
+        if length == 1:
+            self.tok.copy_(ids)
+            self.step()
+            return
+        cfg, L, b = self.cfg, _lib.lib(), self._prefill_buffers()
+        H, F, D = cfg.hidden, cfg.ffn, cfg.head_dim
+        st = _lib.stream_ptr(self.device)
+        c = _lib.check
+        x, o = b["x"], b["o"]
+
+        def norm(src: torch.Tensor, gamma: torch.Tensor, res: torch.Tensor, rows: int) -> None:  # res += norm(src)
+            c(L.bp_decode_norm_residual_rows(src.data_ptr(), gamma.data_ptr(), res.data_ptr(), res.data_ptr(), H, cfg.eps,
+                                             rows, st), "bp_decode_norm_residual_rows")
+
+        def feed_forward(w: dict, res: torch.Tensor, attn: torch.Tensor, rows: int) -> None:
+            self._rows_mm(attn, w["o"], o, rows, H, H, st)
+            norm(o, w["post_attn"], res, rows)
+            if "gu" in b:
+                self._rows_mm(res, w["gate_up"], b["gu"], rows, 2 * F, H, st)
+                c(L.bp_decode_silu_mul_rows(b["gu"].data_ptr(), b["act"].data_ptr(), F, rows, 1, st),
+                  "bp_decode_silu_mul_rows")
+            else:
+                self._rows_mm(res, w["gate_up"], b["act"], rows, 2 * F, H, st, silu=True)
+            self._rows_mm(b["act"], w["down"], o, rows, H, F, st)
+            norm(o, w["post_ff"], res, rows)
+
+        for base in range(0, length, PREFILL_ROWS):
+            rows = min(PREFILL_ROWS, length - base)
+            last_pass = base + rows == length
+            b["ids"][:rows].copy_(ids[base:base + rows])
+            self.pos.fill_(base)
+            c(L.bp_decode_embed_rows(b["ids"].data_ptr(), self.embed.data_ptr(), x.data_ptr(), rows, H, cfg.vocab, st),
+              "bp_decode_embed_rows")
+            for i, w in enumerate(self.layers):
+                kc, vc = self.k_cache[i], self.v_cache[i]
+                self._rows_mm(x, w["qkv"], b["qkv"], rows, 3 * H, H, st)
+                c(L.bp_decode_qk_rope_cache_rows(b["qkv"].data_ptr(), w["q_norm"].data_ptr(), w["k_norm"].data_ptr(),
+                                                 self.inv_freq.data_ptr(), self.pos.data_ptr(), b["q"].data_ptr(),
+                                                 kc.data_ptr(), vc.data_ptr(), cfg.heads, D, cfg.max_len, cfg.eps, rows,
+                                                 st), "bp_decode_qk_rope_cache_rows")
+                top = i + 1 == cfg.layers
+                if top and not last_pass:
+                    break
+                if not top:
+                    c(L.bp_decode_attention_rows(b["q"].data_ptr(), kc.data_ptr(), vc.data_ptr(), self.pos.data_ptr(),
+                                                 b["attn"].data_ptr(), cfg.heads, D, cfg.max_len, self.scale, rows, st),
+                      "bp_decode_attention_rows")
+                    feed_forward(w, x, b["attn"], rows)
+                    continue
+                self.pos.fill_(length - 1)
+                c(L.bp_decode_attention_rows(b["q"][rows - 1].data_ptr(), kc.data_ptr(), vc.data_ptr(),
+                                             self.pos.data_ptr(), self.attn.data_ptr(), cfg.heads, D, cfg.max_len,
+                                             self.scale, 1, st), "bp_decode_attention_rows")
+                feed_forward(w, x[rows - 1:rows], self.attn, 1)
+                c(L.bp_decode_norm_residual(x[rows - 1].data_ptr(), self.norm.data_ptr(), None, self.xn.data_ptr(), H,
+                                            cfg.eps, st), "bp_decode_norm_residual")
+                self._mm(self.xn, self.lm_head, self.logits)
+                c(L.bp_decode_argmax_next(self.logits.data_ptr(), cfg.vocab, self.tok.data_ptr(), self.pos.data_ptr(),
+                                          self.argmax_scratch.data_ptr(), st), "bp_decode_argmax_next")
+
     def argmax_failed(self) -> bool:
         """Whether an argmax launch since the decoder was made gave up waiting for one of its partials (its token
         is then not to be trusted); reads the error words of the argmax scratch (synchronises)."""
@@ -457,10 +561,7 @@ def _loop(dec: OlmoDecoder, group: int, issue: Callable[[int, int], None], prepa
         if min(ids) < 0 or max(ids) >= dec.cfg.vocab:
             raise OptimizeError("token id outside the vocabulary")
         dev = dec.device
-        dec.pos.zero_()
-        for t in ids:  # prefill one position at a time; the last step leaves the first new token in tok
-            dec.tok.fill_(t)
-            dec.step()
+        dec.prefill(inputs[0])  # leaves the first new token in tok
         slots[0].copy_(dec.tok[0], non_blocking=True)
         done[0].record()
         done[0].synchronize()

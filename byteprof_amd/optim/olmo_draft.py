@@ -107,8 +107,8 @@ def make_generate_draft(dec: OlmoDecoder, spec: dict[str, Any] | None = None,
 
     spec: 'kind' ('none' | 'oracle'), 'ks' (draft lengths with a captured graph, default (0, 1, 2, 4, 6, 8)), 'k_max'
     (default 8), 'truth' ({prompt ids tuple: generated tokens}, for 'oracle'), 'drafter' (any object with the
-    protocol). The prompt is fed one position at a time through OlmoDecoder.step (as make_generate does), which
-    also gives the first new token; the rounds then run from the end of the prompt."""
+    protocol). The prompt runs through OlmoDecoder.prefill (as make_generate's), which also gives the first new token; the
+    rounds then run from the end of the prompt."""
     spec = dict(spec or {})
     k_max = int(spec.get("k_max", 8))
     ks = (0,) + tuple(sorted(k for k in spec.get("ks", (0, 1, 2, 4, 6, 8)) if 0 < k <= k_max))
@@ -160,10 +160,7 @@ def make_generate_draft(dec: OlmoDecoder, spec: dict[str, Any] | None = None,
         ids = inputs[0].tolist()
         if min(ids) < 0 or max(ids) >= dec.cfg.vocab:
             raise OptimizeError("token id outside the vocabulary")
-        dec.pos.zero_()
-        for t in ids:  # prefill one position at a time; the last step leaves the first new token in tok
-            dec.tok.fill_(t)
-            dec.step()
+        dec.prefill(inputs[0])  # leaves the first new token in tok
         pinned_one.copy_(dec.tok, non_blocking=True)
         done.record()
         done.synchronize()

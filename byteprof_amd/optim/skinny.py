@@ -401,7 +401,7 @@ def _launch_int4(x: torch.Tensor, w: torch.Tensor, scale: torch.Tensor, zero: to
         ws_bytes = L.bp_skinny_workspace_bytes(m, n, split)
         ws = torch.empty(ws_bytes // 4, dtype=torch.float32, device=x.device)
     rc = L.bp_skinny_int4_rows(x.data_ptr(), w.data_ptr(), scale.data_ptr(), _lib.TORCH_DT[scale.dtype], zero.data_ptr(),
-                               y.data_ptr(), m, n, k, tile_rows, waves, split, _lib.ptr(ws), ws_bytes,
+                               y.data_ptr(), m, n, k, tile_rows, waves, split, 0, _lib.ptr(ws), ws_bytes,
                                _lib.stream_ptr(x.device))
     _lib.check(rc, "bp_skinny_int4_rows")
 

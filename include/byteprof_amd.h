@@ -90,6 +90,14 @@ int64_t bp_skinny_mf_stage_bytes_rows(int wkind, int64_t M, int64_t K, int split
 int bp_skinny_mf(int wkind, const void* x, const void* w, const void* scale, int scale_dtype, void* y, int64_t M,
                  int64_t N, int64_t K, int rb, int waves, int split, int xstage, void* workspace,
                  size_t workspace_bytes, void* stream);
+/* bp_skinny_mf for any number of rows M (a prompt) at the plan (waves, split): one launch of the wide kernel past 64 rows
+ * (with epilogue 1 past 16), each row the bits that bp_skinny_mf gives it. epilogue 0: y [M, N]; 1: the gate|up SiLU
+ * product of bp_skinny_mf_silu, y [M, N] with w [2 N, K] interleaved (split 1). The workspace as for
+ * bp_skinny_workspace_bytes(M, N, split).
+ * Replaces: the linears of the batched prompt forward (byteprof/optim/olmo.py:164-180, HF Olmo2Model). */
+int bp_skinny_mf_rows(int wkind, const void* x, const void* w, const void* scale, int scale_dtype, void* y, int64_t M,
+                      int64_t N, int64_t K, int waves, int split, int epilogue, void* workspace, size_t workspace_bytes,
+                      void* stream);
 /* bp_skinny_mf stopped after the partial sums (split >= 2): workspace [split][M][N] fp32, unscaled for int8 (the
  * reducer applies the scale), e.g. for bp_decode_splitk_norm_residual_rows. */
 int bp_skinny_mf_partials(int wkind, const void* x, const void* w, int64_t M, int64_t N, int64_t K, int rb,
@@ -214,12 +222,12 @@ int bp_skinny_int4_config_supported(int mt, int tile_rows, int waves);
 int bp_skinny_int4(const void* x, const void* packed, const void* scale, int scale_dtype, const void* zero, void* y,
                    int64_t M, int64_t N, int64_t K, int tile_rows, int waves, int split, void* workspace,
                    size_t workspace_bytes, void* stream);
-/* bp_skinny_int4 for 1 <= M <= 64 rows: one launch (skinny_int4_wide.hip) where the matrix-core kernel applies, else one
- * per 16 rows; the same bits as bp_skinny_int4 on each row. Replaces: byteprof/optim/skinny.py:111-133 (_launch) for the
- * row buckets 32 and 64 with MODE 3 weights. */
+/* bp_skinny_int4 for any M: one launch (skinny_int4_wide.hip) where the matrix-core kernel applies, else one per 16 rows;
+ * the same bits as bp_skinny_int4 on each row. epilogue 1: the product of bp_skinny_int4_silu (y [M, N], w [2 N, K]).
+ * Replaces: byteprof/optim/skinny.py:111-133 (_launch) for the row buckets 32 and 64 with MODE 3 weights. */
 int bp_skinny_int4_rows(const void* x, const void* packed, const void* scale, int scale_dtype, const void* zero, void* y,
-                        int64_t M, int64_t N, int64_t K, int tile_rows, int waves, int split, void* workspace,
-                        size_t workspace_bytes, void* stream);
+                        int64_t M, int64_t N, int64_t K, int tile_rows, int waves, int split, int epilogue,
+                        void* workspace, size_t workspace_bytes, void* stream);
 /* bp_skinny_int4 of an interleaved gate|up weight ([2 ffn, K] packed: row 2f the gate row f, row 2f + 1 the up row
  * f) with the SiLU product as the epilogue: out [M, ffn] = bf16(bf16(silu(bf16(g))) * bf16(u)), equal bit for bit to
  * bp_skinny_int4 (same tile rows and waves, split 1) followed by bp_decode_silu_mul_rows (interleaved). The
