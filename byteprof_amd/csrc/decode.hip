@@ -65,32 +65,6 @@ __global__ __launch_bounds__(kBlock) void embed_kernel(const int64_t* __restrict
 }
 
 
-constexpr int kAttnUnroll = 4;  // row batches whose loads are in flight together
-
-// q_row . w_row for 8 bf16 cache values packed in w and 8 q values: the products summed in order.
-__device__ __forceinline__ float dot8(const u32x4& w, const float (&qv)[8]) {
-  const uint32_t wd[4] = {w.x, w.y, w.z, w.w};
-  float dot = 0.f;
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    dot += bf16_bits_to_float(wd[e] & 0xffffu) * qv[2 * e];
-    dot += bf16_bits_to_float(wd[e] >> 16) * qv[2 * e + 1];
-  }
-  return dot;
-}
-
-// Sum of v over each group of LPR consecutive lanes (LPR a power of two <= 32), returned to every lane of the
-// group: DPP pairs within quads, quads within half-rows, half-rows within rows of 16, then rows of 16 in pairs.
-template <int LPR>
-__device__ __forceinline__ float group_sum(float v) {
-  if constexpr (LPR >= 2) v += dpp_f32<0xB1, 0xF>(v);   // quad_perm [1,0,3,2]
-  if constexpr (LPR >= 4) v += dpp_f32<0x4E, 0xF>(v);   // quad_perm [2,3,0,1]
-  if constexpr (LPR >= 8) v += dpp_f32<0x141, 0xF>(v);  // row_half_mirror
-  if constexpr (LPR >= 16) v += dpp_f32<0x140, 0xF>(v); // row_mirror
-  if constexpr (LPR >= 32) v = xor_stage<16>(v, AddOp{});
-  return v;
-}
-
 // Sum (or maximum) of v over the wave, returned to every lane (an xor butterfly, distances 32 .. 1).
 __device__ __forceinline__ float wave_sum(float v) { return xor_butterfly<true>(v, AddOp{}); }
 __device__ __forceinline__ float wave_max(float v) { return xor_butterfly<true>(v, MaxOp{}); }
@@ -98,149 +72,266 @@ __device__ __forceinline__ float wave_max(float v) { return xor_butterfly<true>(
 constexpr int kAttnWaves = kAttnThreads / kWave;
 
 // One head's attention over its cache rows K, V ([max_len, D] bf16, 16-byte aligned, D = 8 * LPR) at positions
-// 0 .. T-1, run by the workgroup's kAttnThreads threads. Layout: LPR lanes per cache row (16 bytes each), 64 / LPR
-// rows per wave instruction, the waves on consecutive rows, and kAttnUnroll such row batches loaded before they
-// are used. The first batch of K and V rows can be loaded early (prefetch(), before the caller's own work), so that
-// its latency overlaps the caller's; a row can be taken from LDS instead of the cache (SUB: the row the caller
-// writes in this launch). Scores: a lane's 8 products in order, then the row's lanes summed (group_sum);
-// s_t = bf16(bf16(q . k_t) * scale), p = bf16(softmax_fp32(s)). Values: each lane accumulates its 8 dimensions
-// over its rows; the row groups of a wave are added by lane butterflies, the waves' sums in wave order through LDS.
-template <int LPR, bool SUB>
-struct HeadAttention {
+// 0 .. T-1, run by the workgroup's kAttnThreads threads: the scores of every position, and the D / S output dimensions
+// of part `part` of S.
+//
+// What bounds it is a CU's own work: a one-row launch has few workgroups, and each took 5 VALU operations a product and
+// 32 KiB of loads in flight (1.9 k positions of 16 heads of 128: 34 us a layer from a cold cache; now 17). So the products
+// are packed (v_dot2_f32_bf16, two of them an operation), a round's reductions share their steps, and S workgroups share
+// a head: each reads the head's whole K rows for the scores (they run on one XCD and meet in its L2), and only its own
+// columns of V. Launches of many rows have workgroups enough (S = 1). The order of every sum is the same for every S:
+//   - scores: LPR lanes per cache row (16 bytes each, whole lines), four row batches per round and the next round's loads
+//     in flight; a lane's 8 products by v_dot2_f32_bf16 in order, then a butterfly over the row's lanes (distances LPR/2
+//     .. 1) for the round's rows at once. s_t = bf16(bf16(q . k_t) * scale), p = bf16(softmax_fp32(s));
+//   - values: position t belongs to class t % C (C = 512 SMAX / LPR). A thread adds its class's positions in order, two
+//     at a time (t and t + C: v_dot2_f32_bf16 on the pair); the classes are added as a tree over the bits of the class:
+//     the highest first (with S = 1 the two classes a thread holds, else a lane bit), then the lowest on, lanes by
+//     butterflies, then waves through LDS.
+// A row can be taken from LDS instead of the cache (SUB: the rows the launch itself writes). RING: the rounds of K rows
+// whose registers a thread holds (1: a launch of many workgroups hides the latency with them, at 64 registers a thread).
+template <int LPR>
+struct AttnShape {
   static constexpr int D = 8 * LPR;
-  static constexpr int RPW = kWave / LPR;           // rows per wave instruction
-  static constexpr int STEP = kAttnWaves * RPW;     // rows per workgroup-wide batch
-  static constexpr int BATCH = kAttnUnroll * STEP;  // rows per round of loads
+  static constexpr int SMAX = LPR >= 8 ? 2 : 1;  // whole lines of the value rows, or half of one
+  static constexpr int C = kAttnThreads * SMAX / LPR;
+  static constexpr int PLEN = kAttnMaxLen + 2 * C;  // scores, then zeros up to whole pairs of classes
+};
+
+// Butterfly over lane distances DIST .. 1 of N values per lane at once (reduce_stage); first: the index of v[0] among the N.
+template <int DIST, int N>
+__device__ __forceinline__ void reduce_rows(float* v, int lane, int& first) {
+  if constexpr (DIST >= 1) {
+    reduce_stage<N, DIST>(v, lane);
+    if constexpr (N > 1) first += (lane & DIST) ? N / 2 : 0;
+    reduce_rows<DIST / 2, (N > 1 ? N / 2 : 1)>(v, lane, first);
+  }
+}
+
+template <int LPR, int S, bool SUB, int RING>
+struct HeadAttention {
+  using A = AttnShape<LPR>;
+  static constexpr int D = A::D, C = A::C;
+  static constexpr int RPW = kWave / LPR;             // K rows per wave instruction
+  static constexpr int STEP = kAttnWaves * RPW;       // K rows per workgroup-wide batch
+  static constexpr int KU = 4;                        // batches per round
+  static constexpr int LV = LPR / S;                  // lanes per value row
+  static constexpr int VSTEP = kAttnThreads / LV;     // value rows per workgroup-wide batch
+  static constexpr int NU = A::SMAX / S;              // classes a thread holds
+  static constexpr int VB = 2 / NU;                   // pairs of C rows per round
+  static constexpr int VU = 2 * NU * VB;              // batches per round
+  static constexpr int PART = kAttnWaves * 8 * LV;    // floats of the value partials
   // the rows 0 .. T-1 of K and V as buffer resources: a row at or past T has an offset past its resource, so its
   // load returns zeros without a memory request (and without a branch around the load)
   __amdgpu_buffer_rsrc_t krs, vrs;
-  int T, s, slot;
-  u32x4 k0[kAttnUnroll], v0[kAttnUnroll];
+  int T, s, slot, vs, vslot, vcol;
+  u32x4 k0[KU], v0[VU];
 
-  __device__ __forceinline__ HeadAttention(const uint16_t* K_, const uint16_t* V_, int T_)
+  __device__ __forceinline__ HeadAttention(const uint16_t* K_, const uint16_t* V_, int T_, int part)
       : krs(buffer_rsrc(K_, 2 * T_ * D)), vrs(buffer_rsrc(V_, 2 * T_ * D)), T(T_) {
     const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
     s = lane % LPR;
     slot = wave * RPW + lane / LPR;  // this lane's row within a batch
+    vs = lane % LV;
+    vslot = slot + (S > 1 ? lane / LV % S * STEP : 0);  // with S = 2, lane bit LV is the class's highest bit
+    vcol = 8 * (LV * part + vs);  // its first output dimension
   }
 
-  __device__ __forceinline__ void load_batch(__amdgpu_buffer_rsrc_t rs, int t0, u32x4 (&out)[kAttnUnroll]) const {
+  // 8 values of row t from column c on
+  __device__ __forceinline__ u32x4 load_row(__amdgpu_buffer_rsrc_t rs, int t, int c) const {
+    const uint32_t off = t < T ? static_cast<uint32_t>(2 * (t * D + c)) : 0x80000000u;
+    return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, off, 0, 0));
+  }
+  __device__ __forceinline__ void load_k(int t0, u32x4 (&out)[KU]) const {
 #pragma unroll
-    for (int u = 0; u < kAttnUnroll; ++u) {
-      const int t = t0 + u * STEP + slot;
-      const uint32_t off = t < T ? static_cast<uint32_t>(2 * (t * D + 8 * s)) : 0x80000000u;
-      out[u] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, off, 0, 0));
-    }
+    for (int u = 0; u < KU; ++u) out[u] = load_row(krs, t0 + u * STEP + slot, 8 * s);
+  }
+  // batch u of a round: class u / (2 VB) ... of pair half u % 2 (the pairs of a class next to each other)
+  __device__ __forceinline__ int vrow(int t0, int u) const {
+    const int half = u % 2, nu = (u / 2) % NU, vb = u / (2 * NU);
+    return t0 + (2 * vb + half) * C + nu * STEP + vslot;
+  }
+  __device__ __forceinline__ void load_v(int t0, u32x4 (&out)[VU]) const {
+#pragma unroll
+    for (int u = 0; u < VU; ++u) out[u] = load_row(vrs, vrow(t0, u), vcol);
   }
 
-  // Issues the loads of the first batch of K and V rows.
+  // Issues the loads of the first round of K and V rows; batches past the end are not issued (even a load that asks for
+  // nothing takes the address unit's time: 1.5 us of 7 at 20 positions).
   __device__ __forceinline__ void prefetch() {
-    load_batch(krs, 0, k0);
-    load_batch(vrs, 0, v0);
-  }
-
-  __device__ __forceinline__ void scores(const u32x4 (&kv)[kAttnUnroll], int t0, const float (&qv)[8],
-                                         const uint16_t* ksub, int sub_lo, float scale, float* sc, float& m) const {
-    float dot[kAttnUnroll];
+    const u32x4 z = u32x4{0u, 0u, 0u, 0u};
 #pragma unroll
-    for (int u = 0; u < kAttnUnroll; ++u) {
-      const int t = t0 + u * STEP + slot;
-      const u32x4 w = SUB && t >= sub_lo && t < T ? *reinterpret_cast<const u32x4*>(ksub + (t - sub_lo) * D + 8 * s)
-                                                  : kv[u];
-      dot[u] = dot8(w, qv);
+    for (int u = 0; u < KU; ++u) {
+      k0[u] = z;
+      if (u * STEP < T) k0[u] = load_row(krs, u * STEP + slot, 8 * s);
     }
 #pragma unroll
-    for (int u = 0; u < kAttnUnroll; ++u) dot[u] = group_sum<LPR>(dot[u]);
+    for (int u = 0; u < VU; ++u) {
+      v0[u] = z;
+      if (vrow(0, u) - vslot < T) v0[u] = load_row(vrs, vrow(0, u), vcol);
+    }
+  }
+
+  __device__ __forceinline__ void scores(const u32x4 (&kv)[KU], int t0, const u32x4& q, const uint16_t* ksub, int sub_lo,
+                                         float scale, float* sc, float& m) const {
+    float dot[KU];
 #pragma unroll
-    for (int u = 0; u < kAttnUnroll; ++u) {
-      const int t = t0 + u * STEP + slot;
+    for (int u = 0; u < KU; ++u) {
+      const int b0 = t0 + u * STEP;  // the batch's first row: the branches are the workgroup's
+      dot[u] = 0.f;
+      if (b0 >= T) continue;
+      u32x4 w = kv[u];
+      if constexpr (SUB) {
+        const int t = b0 + slot;
+        if (b0 + STEP > sub_lo && t >= sub_lo && t < T)
+          w = *reinterpret_cast<const u32x4*>(ksub + (t - sub_lo) * D + 8 * s);
+      }
+      float d = dot2_bf16(w.x, q.x, 0.f);
+      d = dot2_bf16(w.y, q.y, d);
+      d = dot2_bf16(w.z, q.z, d);
+      dot[u] = dot2_bf16(w.w, q.w, d);
+    }
+    const int lane = threadIdx.x % kWave;
+    // each stage halves the rows a lane holds while more than one is left: the lane with bit d set keeps the upper half
+    int first = 0;  // the first row a lane holds at the end, of kLeft
+    reduce_rows<LPR / 2, KU>(dot, lane, first);
+    constexpr int kLeft = KU / (LPR < KU ? LPR : KU);
+#pragma unroll
+    for (int j = 0; j < kLeft; ++j) {
+      const int t = t0 + (first + j) * STEP + slot;
       if (t < T) {
-        const float v = round_to_bf16(round_to_bf16(dot[u]) * scale);
-        if (s == 0) sc[t] = v;
+        const float v = round_to_bf16(round_to_bf16(dot[j]) * scale);
+        sc[t] = v;  // lanes that hold the same row write the same value
         m = fmaxf(m, v);
       }
     }
   }
 
-  __device__ __forceinline__ void values(const u32x4 (&vv)[kAttnUnroll], int t0, const uint16_t* vsub, int sub_lo,
-                                         const float* sc, float inv, float (&acc)[8]) const {
+  __device__ __forceinline__ void values(const u32x4 (&vv)[VU], int t0, const uint16_t* vsub, int sub_lo,
+                                         const float* sc, float inv, float (&acc)[NU][8]) const {
 #pragma unroll
-    for (int u = 0; u < kAttnUnroll; ++u) {
-      const int t = t0 + u * STEP + slot;
+    for (int u = 0; u < VU; u += 2) {
+      const int t = vrow(t0, u);  // and t + C
+      u32x4 a = vv[u], b = vv[u + 1];
+      const int b0 = t - vslot;
+      if (b0 >= T) continue;  // the workgroup's branch
+      if constexpr (SUB) if (b0 + 2 * C > sub_lo) {
+        if (t >= sub_lo && t < T) a = *reinterpret_cast<const u32x4*>(vsub + (t - sub_lo) * D + vcol);
+        if (t + C >= sub_lo && t + C < T) b = *reinterpret_cast<const u32x4*>(vsub + (t + C - sub_lo) * D + vcol);
+      }
       if (t < T) {
-        const u32x4 w = SUB && t >= sub_lo ? *reinterpret_cast<const u32x4*>(vsub + (t - sub_lo) * D + 8 * s) : vv[u];
-        const float p = round_to_bf16(sc[t] * inv);
-        const uint32_t wd[4] = {w.x, w.y, w.z, w.w};
+        const uint32_t p = float_to_bf16_bits(sc[t] * inv) | (static_cast<uint32_t>(float_to_bf16_bits(sc[t + C] * inv)) << 16);
+        float (&ac)[8] = acc[(u / 2) % NU];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          acc[2 * e] += p * bf16_bits_to_float(wd[e] & 0xffffu);
-          acc[2 * e + 1] += p * bf16_bits_to_float(wd[e] >> 16);
+          ac[2 * e] = dot2_bf16(__builtin_amdgcn_perm(b[e], a[e], 0x05040100u), p, ac[2 * e]);
+          ac[2 * e + 1] = dot2_bf16(__builtin_amdgcn_perm(b[e], a[e], 0x07060302u), p, ac[2 * e + 1]);
         }
       }
     }
   }
 
-  // q: bf16 values in LDS qs[0 .. D). Rows t >= sub_lo (INT_MAX: none) are read from ksub / vsub [t - sub_lo][D]
-  // (bf16, LDS, 16-byte aligned rows) instead of the cache. Writes out[0 .. D). The caller has made qs, ksub and
-  // vsub visible (a barrier).
-  // LDS: sc[T] scores, red_m / red_l [kAttnWaves], part [kAttnWaves * D].
-  __device__ __forceinline__ void run(const float* qs, const uint16_t* ksub, const uint16_t* vsub, int sub_lo,
-                                      float scale, float* sc, float* red_m, float* red_l, float* part,
+  // q: bf16 values in LDS qs[0 .. D) (16-byte aligned). Rows t >= sub_lo (INT_MAX: none) are read from ksub / vsub
+  // [t - sub_lo][D] (bf16, LDS, 16-byte aligned rows) instead of the cache. Writes out[0 .. D)'s part. The caller has made
+  // qs, ksub and vsub visible (a barrier). LDS: sc[PLEN] scores, part_sums[PART], red_m / red_l [kAttnWaves].
+  __device__ __forceinline__ void run(const uint16_t* qs, const uint16_t* ksub, const uint16_t* vsub, int sub_lo,
+                                      float scale, float* sc, float* part_sums, float* red_m, float* red_l,
                                       uint16_t* __restrict__ out) {
     const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
-    float qv[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) qv[e] = qs[8 * s + e];
+    const u32x4 q = *reinterpret_cast<const u32x4*>(qs + 8 * s);
     float m = -INFINITY;
-    scores(k0, 0, qv, ksub, sub_lo, scale, sc, m);
-    for (int t0 = BATCH; t0 < T; t0 += BATCH) {
-      u32x4 kv[kAttnUnroll];
-      load_batch(krs, t0, kv);
-      scores(kv, t0, qv, ksub, sub_lo, scale, sc, m);
+    constexpr int R = KU * STEP;
+    if constexpr (RING == 1) {
+      scores(k0, 0, q, ksub, sub_lo, scale, sc, m);
+      for (int t0 = R; t0 < T; t0 += R) {
+        load_k(t0, k0);
+        scores(k0, t0, q, ksub, sub_lo, scale, sc, m);
+      }
+    } else {
+      // often few positions: the next round's loads only where there is one (a load past the end costs
+      // the address unit's time), each case on its own path, so that the waits stay exact
+      u32x4 k1[KU];
+      for (int t0 = 0;; t0 += 2 * R) {
+        if (t0 + R >= T) {
+          scores(k0, t0, q, ksub, sub_lo, scale, sc, m);
+          break;
+        }
+        load_k(t0 + R, k1);
+        scores(k0, t0, q, ksub, sub_lo, scale, sc, m);
+        if (t0 + 2 * R >= T) {
+          scores(k1, t0 + R, q, ksub, sub_lo, scale, sc, m);
+          break;
+        }
+        load_k(t0 + 2 * R, k0);
+        scores(k1, t0 + R, q, ksub, sub_lo, scale, sc, m);
+      }
     }
+    constexpr int RV = 2 * VB * C;
+    u32x4 v1[RING > 1 ? VU : 1];
+    if constexpr (RING > 1)
+      if (T > RV) load_v(RV, v1);  // in flight during the softmax
     m = wave_max(m);
     if (lane == 0) red_m[wave] = m;
     __syncthreads();  // also orders the sc writes before the reads below
     m = red_m[0];
     for (int w = 1; w < kAttnWaves; ++w) m = fmaxf(m, red_m[w]);
     float l = 0.f;
-    for (int t = threadIdx.x; t < T; t += kAttnThreads) {
-      const float e = expf(sc[t] - m);
+    const int tend = (T + 2 * C - 1) / (2 * C) * (2 * C);  // zeros up to whole pairs of classes
+    for (int t = threadIdx.x; t < tend; t += kAttnThreads) {
+      const float e = t < T ? expf(sc[t] - m) : 0.f;
       sc[t] = e;
       l += e;
     }
     l = wave_sum(l);
     if (lane == 0) red_l[wave] = l;
-    __syncthreads();  // also orders the sc writes before the reads below
+    __syncthreads();
     l = red_l[0];
     for (int w = 1; w < kAttnWaves; ++w) l += red_l[w];
     const float inv = 1.f / l;
-    float acc[8];
+    float acc[NU][8];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) acc[e] = 0.f;
-    values(v0, 0, vsub, sub_lo, sc, inv, acc);
-    for (int t0 = BATCH; t0 < T; t0 += BATCH) {
-      u32x4 vv[kAttnUnroll];
-      load_batch(vrs, t0, vv);
-      values(vv, t0, vsub, sub_lo, sc, inv, acc);
+    for (int u = 0; u < NU; ++u)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) acc[u][e] = 0.f;
+    if constexpr (RING == 1) {
+      values(v0, 0, vsub, sub_lo, sc, inv, acc);
+      for (int t0 = RV; t0 < T; t0 += RV) {
+        load_v(t0, v0);
+        values(v0, t0, vsub, sub_lo, sc, inv, acc);
+      }
+    } else {
+      for (int t0 = 0;; t0 += 2 * RV) {
+        values(v0, t0, vsub, sub_lo, sc, inv, acc);
+        if (t0 + RV >= T) break;
+        if (t0 + 2 * RV >= T) {
+          values(v1, t0 + RV, vsub, sub_lo, sc, inv, acc);
+          break;
+        }
+        load_v(t0 + 2 * RV, v0);
+        values(v1, t0 + RV, vsub, sub_lo, sc, inv, acc);
+        if (t0 + 3 * RV < T) load_v(t0 + 3 * RV, v1);
+      }
     }
-    // the wave's row groups (lanes s, s + LPR, s + 2 LPR, ...) added by butterflies over the group bits
+    // the thread's classes, then the wave's lanes (lane bits LV ..)
 #pragma unroll
-    for (int e = 0; e < 8; ++e) acc[e] = xor_butterfly<false, LPR>(acc[e], AddOp{});
-    if (lane < LPR) {
+    for (int e = 0; e < 8; ++e) {
+      if constexpr (NU == 2) acc[0][e] += acc[1][e];
+      acc[0][e] = xor_butterfly<false, LV>(acc[0][e], AddOp{});
+    }
+    if (lane < LV) {
 #pragma unroll
-      for (int e = 0; e < 8; ++e) part[wave * D + 8 * s + e] = acc[e];
+      for (int e = 0; e < 8; ++e) part_sums[wave * (8 * LV) + 8 * vs + e] = acc[0][e];
     }
     __syncthreads();
-    for (int d = threadIdx.x; d < D; d += kAttnThreads) {
-      float t = part[d];
-      for (int w = 1; w < kAttnWaves; ++w) t += part[w * D + d];
-      out[d] = float_to_bf16_bits(t);
+    const int col0 = vcol - 8 * vs;
+    for (int d = threadIdx.x; d < 8 * LV; d += kAttnThreads) {
+      float w8[kAttnWaves];
+#pragma unroll
+      for (int w = 0; w < kAttnWaves; ++w) w8[w] = part_sums[w * (8 * LV) + d];
+      out[col0 + d] = float_to_bf16_bits(((w8[0] + w8[1]) + (w8[2] + w8[3])) + ((w8[4] + w8[5]) + (w8[6] + w8[7])));
     }
   }
 };
-
-constexpr int kAttnPart = kAttnWaves * 256;  // floats of the value partials: waves x D (D <= 256)
+static_assert(kAttnWaves == 8, "the tree over the waves");
 
 // 1 / rms of q[0 .. H) and of k[0 .. H) (+ eps inside the root), by a kAttnThreads-thread workgroup: thread t sums
 // the squares of elements 8t .. 8t + 7 (then + 8 * kAttnThreads ...) in order, each wave by a butterfly, the waves in
@@ -281,10 +372,9 @@ __device__ __forceinline__ void qk_rms(const uint16_t* q, const uint16_t* k, int
 }
 
 // The RoPE pair (a, a + D/2) of head h at position pos: q and k normalised (weights in fp32, bf16 rounding), rotated
-// with fp32 cos / sin; returns the rotated q as bf16 values and k as bf16 bits.
+// with fp32 cos / sin; returns the rotated q and k as bf16 bits.
 struct RopePair {
-  float qa, qb;
-  uint16_t ka, kb;
+  uint16_t qa, qb, ka, kb;
 };
 __device__ __forceinline__ RopePair rope_pair(float fqa, float fqb, float fka, float fkb, float wqa, float wqb,
                                               float wka, float wkb, float fr, int64_t pos, float rq, float rk) {
@@ -295,8 +385,8 @@ __device__ __forceinline__ RopePair rope_pair(float fqa, float fqb, float fka, f
   const float ka = round_to_bf16(wka * (fka * rk));
   const float kb = round_to_bf16(wkb * (fkb * rk));
   RopePair r;
-  r.qa = round_to_bf16(qa * c + (-qb) * sn);
-  r.qb = round_to_bf16(qb * c + qa * sn);
+  r.qa = float_to_bf16_bits(qa * c + (-qb) * sn);
+  r.qb = float_to_bf16_bits(qb * c + qa * sn);
   r.ka = float_to_bf16_bits(ka * c + (-kb) * sn);
   r.kb = float_to_bf16_bits(kb * c + ka * sn);
   return r;
@@ -329,8 +419,8 @@ __global__ __launch_bounds__(kAttnThreads) void qk_rope_cache_kernel(const uint1
     const int a = h * D + j, b = a + half;
     const RopePair rp = rope_pair(ld_bf16(q, a), ld_bf16(q, b), ld_bf16(k, a), ld_bf16(k, b), ld_bf16(qw, a),
                                   ld_bf16(qw, b), ld_bf16(kw, a), ld_bf16(kw, b), inv_freq[j], pos, rq, rk);
-    qo[a] = float_to_bf16_bits(rp.qa);
-    qo[b] = float_to_bf16_bits(rp.qb);
+    qo[a] = rp.qa;
+    qo[b] = rp.qb;
     if (in_cache) {
       const int64_t row = (static_cast<int64_t>(h) * max_len + pos) * D;
       kc[row + j] = rp.ka;
@@ -344,32 +434,59 @@ __global__ __launch_bounds__(kAttnThreads) void qk_rope_cache_kernel(const uint1
 // grid = (heads, rows); row r of q / out [rows, heads * D] attends over positions 0 .. *pos_p + r of the head's
 // cache rows [max_len, D], D = 8 * LPR.
 template <int LPR>
-__global__ __launch_bounds__(kAttnThreads) void attention_kernel(const uint16_t* __restrict__ q,
+__global__ __launch_bounds__(kAttnThreads, 8) void attention_kernel(const uint16_t* __restrict__ q,
                                                                  const uint16_t* __restrict__ kc,
                                                                  const uint16_t* __restrict__ vc,
                                                                  const int64_t* __restrict__ pos_p,
                                                                  uint16_t* __restrict__ out, int max_len,
                                                                  float scale) {
   constexpr int D = 8 * LPR;
-  __shared__ float sc[kAttnMaxLen];
-  __shared__ float qs[D];
+  using Att = HeadAttention<LPR, 1, false, 1>;
+  __shared__ float sc[AttnShape<LPR>::PLEN];
+  __shared__ float part[Att::PART];
+  __shared__ __align__(16) uint16_t qs[D];
   __shared__ float red_m[kAttnWaves], red_l[kAttnWaves];
-  __shared__ float part[kAttnPart];
   const int h = blockIdx.x, r = blockIdx.y;
   const int64_t row = (static_cast<int64_t>(r) * gridDim.x + h) * D;
   int64_t pos = *pos_p + r;
   pos = pos < 0 ? 0 : (pos >= max_len ? max_len - 1 : pos);
-  HeadAttention<LPR, false> att(kc + static_cast<int64_t>(h) * max_len * D,
-                                vc + static_cast<int64_t>(h) * max_len * D, static_cast<int>(pos) + 1);
+  Att att(kc + static_cast<int64_t>(h) * max_len * D, vc + static_cast<int64_t>(h) * max_len * D,
+          static_cast<int>(pos) + 1, 0);
   att.prefetch();
-  for (int d = threadIdx.x; d < D; d += kAttnThreads) qs[d] = ld_bf16(q, row + d);
+  for (int d = threadIdx.x; d < D; d += kAttnThreads) qs[d] = q[row + d];
   __syncthreads();
-  att.run(qs, nullptr, nullptr, INT_MAX, scale, sc, red_m, red_l, part, out + row);
+  att.run(qs, nullptr, nullptr, INT_MAX, scale, sc, part, red_m, red_l, out + row);
 }
 
-// qk_rope_cache and attention in one launch: every workgroup h computes the q / k norms over the whole projections
+// A one-row launch of long contexts has few workgroups, so its reads from memory are bounded by the loads that those keep
+// in flight. kAttnReaders more workgroups per head, on the head's XCD, each read a share of the T cache rows and use
+// nothing of them: the lines are in that XCD's L2 when the head's own workgroups come to them. From kReadFrom positions
+// on (below, the first rounds of loads cover most of the cache). 16 heads of 128 at 4000 positions: 36 us a layer without
+// them, 30 with; eight cold layers at 1900 positions 172 us without, 137 with.
+constexpr int kAttnReaders = 8;
+constexpr int kReadFrom = 512;
+template <int D>
+__device__ __forceinline__ void read_rows(const uint16_t* K, const uint16_t* V, int T, int share) {
+  if (T < kReadFrom) return;
+  const int lo = static_cast<int>(static_cast<int64_t>(T) * share / kAttnReaders) * (D / 8);  // in 16-byte pieces
+  const int hi = static_cast<int>(static_cast<int64_t>(T) * (share + 1) / kAttnReaders) * (D / 8);
+  const auto k = as_global(reinterpret_cast<const u32x4*>(K)), v = as_global(reinterpret_cast<const u32x4*>(V));
+  for (int i = lo + static_cast<int>(threadIdx.x); i < hi; i += 4 * kAttnThreads) {
+    u32x4 a[4], b[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int e = min(i + u * kAttnThreads, hi - 1);
+      a[u] = k[e];
+      b[u] = v[e];
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) asm volatile("" ::"v"(a[u]), "v"(b[u]));  // the loads stay
+  }
+}
+
+// qk_rope_cache and attention in one launch, SMAX workgroups per head (HeadAttention): every workgroup computes the q / k norms over the whole projections
 // (the same sums in every workgroup, in qk_rope_cache_kernel's order: the results are equal bit for bit to the two
-// launches), rotates its own head, writes its k and v at pos to the cache, and attends over positions
+// launches), rotates its own head, the first of a head writes its k and v at pos to the cache, and each attends over positions
 // 0 .. pos with that row taken from LDS. Every load that does not depend on the norms (the projections, the RoPE
 // operands, the first batch of cache rows) is issued before the first reduction.
 template <int LPR>
@@ -384,13 +501,19 @@ __global__ __launch_bounds__(kAttnThreads) void rope_attention_kernel(const uint
                                                                       int max_len, float eps, float scale) {
   constexpr int D = 8 * LPR;
   constexpr int half = D / 2;
-  __shared__ float sc[kAttnMaxLen];
-  __shared__ float qs[D];
+  constexpr int S = AttnShape<LPR>::SMAX;
+  using Att = HeadAttention<LPR, S, true, 2>;
+  __shared__ float sc[AttnShape<LPR>::PLEN];
+  __shared__ float part[Att::PART];
+  __shared__ __align__(16) uint16_t qs[D];
   __shared__ __align__(16) uint16_t ks[D];
   __shared__ __align__(16) uint16_t vs[D];
   __shared__ float red_q[kAttnWaves], red_k[kAttnWaves], red_m[kAttnWaves], red_l[kAttnWaves];
-  __shared__ float part[kAttnPart];
-  const int h = blockIdx.x;
+  // the workgroups of a head 8 apart, on one XCD (workgroups go to the 8 XCDs in turn): its S parts, then the readers
+  constexpr int kWgs = kXcds * (S + kAttnReaders);
+  const int grp = blockIdx.x / kWgs, in = blockIdx.x % kWgs;
+  const int h = grp * kXcds + in % kXcds, vpart = in / kXcds;
+  if (h >= heads) return;  // the last group's missing heads (the whole workgroup)
   const int H = heads * D;
   const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
   const int64_t pos_in = *pos_p;
@@ -401,6 +524,10 @@ __global__ __launch_bounds__(kAttnThreads) void rope_attention_kernel(const uint
   const uint16_t* v = qkv + 2 * H;
   uint16_t* K = kc + static_cast<int64_t>(h) * max_len * D;
   uint16_t* V = vc + static_cast<int64_t>(h) * max_len * D;
+  if (vpart >= S) {
+    read_rows<D>(K, V, static_cast<int>(pos), vpart - S);
+    return;
+  }
 
   // RoPE operands of this thread's pair (j, j + D/2) of head h (threads j < D/2; D <= 256 <= threads)
   const int j = threadIdx.x;
@@ -421,7 +548,7 @@ __global__ __launch_bounds__(kAttnThreads) void rope_attention_kernel(const uint
     v_b = v[b];
     fr = inv_freq[j];
   }
-  HeadAttention<LPR, true> att(K, V, static_cast<int>(pos) + 1);
+  Att att(K, V, static_cast<int>(pos) + 1, vpart);
   att.prefetch();
 
   // the norms over the whole projections
@@ -437,7 +564,7 @@ __global__ __launch_bounds__(kAttnThreads) void rope_attention_kernel(const uint
     ks[j + half] = k_hi;
     vs[j] = v_a;
     vs[j + half] = v_b;
-    if (in_cache) {
+    if (in_cache && vpart == 0) {
       const int64_t r = pos_in * D;
       K[r + j] = k_lo;
       K[r + j + half] = k_hi;
@@ -446,7 +573,7 @@ __global__ __launch_bounds__(kAttnThreads) void rope_attention_kernel(const uint
     }
   }
   __syncthreads();  // qs, ks and vs, written above, are read below
-  att.run(qs, ks, vs, in_cache ? static_cast<int>(pos_in) : INT_MAX, scale, sc, red_m, red_l, part,
+  att.run(qs, ks, vs, in_cache ? static_cast<int>(pos_in) : INT_MAX, scale, sc, part, red_m, red_l,
           out + static_cast<int64_t>(h) * D);
 }
 
@@ -469,12 +596,13 @@ __global__ __launch_bounds__(kAttnThreads) void rope_attention_rows_kernel(const
                                                                            int max_len, float eps, float scale) {
   constexpr int D = 8 * LPR;
   constexpr int half = D / 2;
-  __shared__ float sc[kAttnMaxLen];
-  __shared__ float qs[D];
+  using Att = HeadAttention<LPR, 1, true, 2>;
+  __shared__ float sc[AttnShape<LPR>::PLEN];
+  __shared__ float part[Att::PART];
+  __shared__ __align__(16) uint16_t qs[D];
   __shared__ __align__(16) uint16_t ks[kRowsMax * D];
   __shared__ __align__(16) uint16_t vs[kRowsMax * D];
   __shared__ float red_q[kAttnWaves], red_k[kRowsMax][kAttnWaves], red_m[kAttnWaves], red_l[kAttnWaves];
-  __shared__ float part[kAttnPart];
   const int h = blockIdx.x, r = blockIdx.y;
   const int H = heads * D;
   const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
@@ -484,7 +612,7 @@ __global__ __launch_bounds__(kAttnThreads) void rope_attention_rows_kernel(const
   const int64_t posc = pos_r < 0 ? 0 : (pos_r >= max_len ? max_len - 1 : pos_r);
   uint16_t* K = kc + static_cast<int64_t>(h) * max_len * D;
   uint16_t* V = vc + static_cast<int64_t>(h) * max_len * D;
-  HeadAttention<LPR, true> att(K, V, static_cast<int>(posc) + 1);
+  Att att(K, V, static_cast<int>(posc) + 1, 0);
   att.prefetch();
 
   // RoPE operands of this thread's (row, pair) items: item i = threadIdx.x + p * kAttnThreads is pair i % (D/2) of
@@ -587,7 +715,7 @@ __global__ __launch_bounds__(kAttnThreads) void rope_attention_rows_kernel(const
   const int64_t lo = pos0 < 0 ? 0 : pos0;
   const bool sub = lo <= pos_r && lo < max_len;
   const int64_t off = sub ? (lo - pos0) * D : 0;
-  att.run(qs, ks + off, vs + off, sub ? static_cast<int>(lo) : INT_MAX, scale, sc, red_m, red_l, part,
+  att.run(qs, ks + off, vs + off, sub ? static_cast<int>(lo) : INT_MAX, scale, sc, part, red_m, red_l,
           out + static_cast<int64_t>(r) * H + static_cast<int64_t>(h) * D);
 }
 
@@ -606,7 +734,8 @@ void launch_rope_attention(const void* qkv, const void* qw, const void* kw, cons
                            void* kc, void* vc, void* out, int heads, int rows, int max_len, float eps, float scale,
                            hipStream_t st) {
   if (rows == 1) {
-    rope_attention_kernel<LPR><<<heads, kAttnThreads, 0, st>>>(
+    constexpr int kGroup = kXcds * (AttnShape<LPR>::SMAX + kAttnReaders);
+    rope_attention_kernel<LPR><<<(heads + kXcds - 1) / kXcds * kGroup, kAttnThreads, 0, st>>>(
         static_cast<const uint16_t*>(qkv), static_cast<const uint16_t*>(qw), static_cast<const uint16_t*>(kw),
         inv_freq, pos, static_cast<uint16_t*>(kc), static_cast<uint16_t*>(vc), static_cast<uint16_t*>(out), heads,
         max_len, eps, scale);
