@@ -199,6 +199,36 @@ __device__ __forceinline__ void mf_wait_vm() {
   __builtin_amdgcn_s_waitcnt((n & 0xF) | ((n >> 4) << 14) | (0x7 << 4) | (0xF << 8));
 }
 
+// What turns a loaded 16 bytes of weights into the lane's MFMA operand. MfInOrder: nothing (the load was in operand order:
+// lane (g, i) reads row i % 8, piece 2 g + i / 8). MfPatch: the load was in memory order (lane l reads row l / 8, piece
+// l % 8, eight neighbouring lanes one 128-byte line) and goes through the wave's own 1 KiB LDS patch: a load whose
+// neighbouring lanes are in different rows takes the address unit four times as long, about 64 cycles a KiB, and a CU
+// that took its weights and activations so was bound by that, not by memory (2048 x 8192 bf16 at one row took 8.3 us from
+// memory and 8.2 from the caches; in memory order 7.8; at 8 rows 10.9 and 9.3). Piece p of row r lies at p ^ (r & 6), so that neither the
+// row-wise writes nor the operand reads conflict; the wave's LDS operations run in order, so no barrier is needed.
+struct MfInOrder {
+  MfInOrder() = default;
+  __device__ __forceinline__ MfInOrder(const uint8_t*, int) {}
+  __device__ __forceinline__ u32x4 operator()(const u32x4& w) const { return w; }
+};
+struct MfPatch {
+  uint8_t* st;
+  const uint8_t* ld;
+  __device__ __forceinline__ MfPatch(uint8_t* patch, int lane) {
+    const MfLane ln(lane);
+    const int r = lane >> 3;
+    st = patch + r * 128 + 16 * ((lane & 7) ^ (r & 6));
+    ld = patch + ln.r * 128 + 16 * (ln.slot() ^ (ln.r & 6));
+  }
+  __device__ __forceinline__ u32x4 operator()(const u32x4& w) const {
+    *reinterpret_cast<u32x4*>(st) = w;
+    __builtin_amdgcn_wave_barrier();
+    const u32x4 v = *reinterpret_cast<const u32x4*>(ld);
+    __builtin_amdgcn_wave_barrier();
+    return v;
+  }
+};
+
 // No-op hook of MfMain::run.
 struct MfNoHook {
   __device__ __forceinline__ void operator()() const {}
@@ -234,39 +264,44 @@ struct MfMain {
   }
 
   // The MFMAs of segment s (its weights in the slot) into the wave's tiles.
+  template <class Turn>
   __device__ __forceinline__ static void compute_slot(const Slot& sl, const XS& xs, int64_t s,
-                                                      floatx4 (&acc)[RB][MB]) {
+                                                      floatx4 (&acc)[RB][MB], const Turn& turn) {
+    u32x4 bx[MB * G::kParts];  // read once for all row blocks (the weights' pass through LDS is in the compiler's way)
+#pragma unroll
+    for (int b = 0; b < MB; ++b)
+#pragma unroll
+      for (int p = 0; p < G::kParts; ++p) {
+        if constexpr (XMEM) {
+          bx[b * G::kParts + p] = sl.x[b * G::kParts + p];
+        } else {
+          bx[b * G::kParts + p] = xs.load(s, b, p);
+        }
+      }
 #pragma unroll
     for (int rb = 0; rb < RB; ++rb) {
+      const u32x4 wv = turn(sl.w[rb]);
       u32x4 a[G::kParts];
       if constexpr (KIND == kBf16) {
-        a[0] = sl.w[rb];
+        a[0] = wv;
       } else {
-        a[0] = mf_i8x8(sl.w[rb].x, sl.w[rb].y);
-        a[1] = mf_i8x8(sl.w[rb].z, sl.w[rb].w);
+        a[0] = mf_i8x8(wv.x, wv.y);
+        a[1] = mf_i8x8(wv.z, wv.w);
       }
 #pragma unroll
       for (int b = 0; b < MB; ++b)
 #pragma unroll
-        for (int p = 0; p < G::kParts; ++p) {
-          u32x4 bx;
-          if constexpr (XMEM) {
-            bx = sl.x[b * G::kParts + p];
-          } else {
-            bx = xs.load(s, b, p);
-          }
-          acc[rb][b] = mf_mfma(a[p], bx, acc[rb][b]);
-        }
+        for (int p = 0; p < G::kParts; ++p) acc[rb][b] = mf_mfma(a[p], bx[b * G::kParts + p], acc[rb][b]);
     }
   }
 
   // wrow[rb]: the lane's weight row of block rb, advanced to the lane's byte offset in a segment.
   // (VEC = false: wrow[rb] is the row start and kl the lane's K offset in a segment, for bounded element loads.)
-  template <class Hook = MfNoHook, class First = MfNoHook>
+  template <class Hook = MfNoHook, class First = MfNoHook, class Turn = MfInOrder>
   __device__ __forceinline__ static void run(const uint8_t* const (&wrow)[RB], const XS& xs, const void* ph,
                                              int64_t K, int64_t kl, int64_t s_first, int64_t stride, int64_t nseg,
                                              floatx4 (&acc)[RB][MB], const Hook& hook = Hook(),
-                                             const First& first = First()) {
+                                             const First& first = First(), const Turn& turn = Turn()) {
     Slot buf[D];
     auto issue = [&](Slot& sl, int64_t idx) {
       const bool live = idx < nseg;
@@ -300,7 +335,7 @@ struct MfMain {
       do {
 #pragma unroll
         for (int d = 0; d < D; ++d) {
-          compute_slot(buf[d], xs, s_first + (base + d) * stride, acc);
+          compute_slot(buf[d], xs, s_first + (base + d) * stride, acc, turn);
           if (d == 0 && base == 0) first();
           issue(buf[d], base + d + D);
           if constexpr (VEC) __builtin_amdgcn_sched_barrier(0);
@@ -310,7 +345,7 @@ struct MfMain {
     }
 #pragma unroll
     for (int d = 0; d < D; ++d) {
-      if (base + d < nseg) compute_slot(buf[d], xs, s_first + (base + d) * stride, acc);
+      if (base + d < nseg) compute_slot(buf[d], xs, s_first + (base + d) * stride, acc, turn);
       if (d == 0 && base == 0) first();
     }
   }
@@ -325,17 +360,17 @@ struct MfFixed {
   using Ops = MfMain<KIND, MB, RB, 1, true, XMEM, XS>;
   static constexpr int kD = D < NSEG ? D : NSEG;  // segments in flight
 
-  template <class Hook = MfNoHook, class First = MfNoHook>
+  template <class Hook = MfNoHook, class First = MfNoHook, class Turn = MfInOrder>
   __device__ __forceinline__ static void run(const uint8_t* const (&wrow)[RB], const XS& xs, int64_t s_first,
                                              int64_t stride, floatx4 (&acc)[RB][MB], const Hook& hook = Hook(),
-                                             const First& first = First()) {
+                                             const First& first = First(), const Turn& turn = Turn()) {
     typename Ops::Slot buf[kD];
 #pragma unroll
     for (int i = 0; i < kD; ++i) Ops::load_slot(buf[i], wrow, xs, s_first + i * stride);
     hook();
 #pragma unroll
     for (int i = 0; i < NSEG; ++i) {
-      Ops::compute_slot(buf[i % kD], xs, s_first + i * stride, acc);
+      Ops::compute_slot(buf[i % kD], xs, s_first + i * stride, acc, turn);
       if (i == 0) first();
       if (i + kD < NSEG) Ops::load_slot(buf[i % kD], wrow, xs, s_first + (i + kD) * stride);
     }

@@ -8,6 +8,7 @@
 #pragma once
 
 #include <algorithm>
+#include <type_traits>
 
 #include "byteprof_amd.h"
 #include "skinny_mf.h"
@@ -185,11 +186,16 @@ __global__ __launch_bounds__(WAVES * WR * kWave) void skinny_mf_kernel(const uin
   static_assert(NSEG == 0 || VEC, "the fixed segment count needs vector loads");
   static_assert(WR == 1 || (XL && !PRO), "row groups share the staged activations (no prologue)");
   constexpr int NW = WAVES * WR;  // the workgroup's waves
+  // Weights in memory order through the LDS patch, except where the LDS has more to do than the address unit: int8 with
+  // staged activations of up to 8 rows or four row blocks a wave (us in order / through the patch: 100352 x 2048 at one
+  // row, staged, 33.9 / 35.0; 16384 x 2048, four blocks, 8.4 / 9.0; but 2048 x 2048 at 4 rows, two blocks, 4.2 / 3.6).
+  constexpr bool kPatch = VEC && !(KIND == kInt8 && ((XL && MB == 1) || RB == 4));
   constexpr int NT = NW * kWave;
   constexpr int D = VEC ? mf_depth<KIND, MB, RB, !XL>() : 1;
   constexpr int kInFlight = NSEG > 0 && NSEG < D ? NSEG : D;  // weight segments issued before the staging commit
   __shared__ MfRed<WAVES, RB, MB> red[WR];
   __shared__ float pro_sums[PRO ? 8 * MB : 1];  // the prologue's per-row sums of squares
+  __shared__ __align__(16) uint8_t patch[kPatch ? NW : 1][1024];  // the waves' weight patches (MfPatch)
   extern __shared__ __attribute__((aligned(16))) uint16_t xs_lds[];
 
 #ifdef BP_TIMELINE
@@ -251,14 +257,16 @@ __global__ __launch_bounds__(WAVES * WR * kWave) void skinny_mf_kernel(const uin
   const int64_t nseg = NSEG > 0 ? NSEG : mf_uniform(s_first < s_hi ? (s_hi - s_first + WAVES - 1) / WAVES : 0);
 
   // the lane's weight rows (rows past N read row N - 1; their outputs are never stored), advanced to the lane's
-  // 16 bytes of a segment (VEC = false: the row start; the element loads add the lane's K offset kl)
+  // 16 bytes of a segment, in memory order for MfPatch, else in operand order (VEC = false: the row start; the element
+  // loads add the lane's K offset kl)
   const int64_t kl = static_cast<int64_t>(G::kLaneK) * ln.slot();
   const uint8_t* wrow[RB];
 #pragma unroll
   for (int rb = 0; rb < RB; ++rb) {
-    const int64_t row = std::min<int64_t>(n0 + 8 * rb + ln.r, N - 1);
-    wrow[rb] = w + row * K * G::kEB + (VEC ? 16 * ln.slot() : 0);
+    const int64_t row = std::min<int64_t>(n0 + 8 * rb + (kPatch ? lane >> 3 : ln.r), N - 1);
+    wrow[rb] = w + row * K * G::kEB + (VEC ? 16 * (kPatch ? lane & 7 : ln.slot()) : 0);
   }
+  const std::conditional_t<kPatch, MfPatch, MfInOrder> turn(patch[kPatch ? wave : 0], lane);
   floatx4 acc[RB][MB];
 #pragma unroll
   for (int rb = 0; rb < RB; ++rb)
@@ -351,20 +359,20 @@ __global__ __launch_bounds__(WAVES * WR * kWave) void skinny_mf_kernel(const uin
       MF_TL(1);
     };
     if constexpr (NSEG > 0)
-      MfFixed<KIND, MB, RB, D, NSEG, false, MfXLds<KIND, MB>>::run(wrow, xs, s_first, WAVES, acc, commit, first);
+      MfFixed<KIND, MB, RB, D, NSEG, false, MfXLds<KIND, MB>>::run(wrow, xs, s_first, WAVES, acc, commit, first, turn);
     else
       MfMain<KIND, MB, RB, D, true, false, MfXLds<KIND, MB>>::run(wrow, xs, x, K, kl, s_first, WAVES, nseg, acc,
-                                                                 commit, first);
+                                                                 commit, first, turn);
   } else if constexpr (VEC) {
     MfXGlobal<KIND, MB, true> xs;
     xs.init(x, M, K, ln);
     const auto issued = [&]() { MF_TL(1); };
     if constexpr (NSEG > 0)
       MfFixed<KIND, MB, RB, D, NSEG, true, MfXGlobal<KIND, MB, true>>::run(wrow, xs, s_first, WAVES, acc, issued,
-                                                                           first);
+                                                                           first, turn);
     else
       MfMain<KIND, MB, RB, D, true, true, MfXGlobal<KIND, MB, true>>::run(wrow, xs, x, K, kl, s_first, WAVES, nseg,
-                                                                          acc, issued, first);
+                                                                          acc, issued, first, turn);
   } else {
     // element loads with bounds (K not a multiple of the segment or unaligned operands): same segments, same order
     MfXGlobal<KIND, MB, false> xs;
