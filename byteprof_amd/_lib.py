@@ -146,8 +146,9 @@ def check(status: int, what: str) -> None:
 
 
 def stream_ptr(device: torch.device) -> int:
-    """hipStream_t of torch's current stream on `device`, as an integer."""
-    return torch.cuda.current_stream(device).cuda_stream
+    """hipStream_t of torch's current stream on `device`, as an integer (without building a Stream object)."""
+    index = device.index
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
 
 
 def ptr(t: torch.Tensor | None) -> int | None:
