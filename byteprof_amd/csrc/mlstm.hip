@@ -68,6 +68,11 @@ __device__ __forceinline__ void store_io(void* p, int64_t i, float f) {
   else static_cast<float*>(p)[i] = f;
 }
 
+// Makes f a value the compiler cannot see through. A launch of one position reads its fp16 state only rounded, and there
+// the compiler makes the multiply-add and the rounding one instruction (v_fma_mixlo_f16, which rounds once): other bits
+// than the fp32 state rounded to fp16, which is what the same position of a longer launch gives.
+__device__ __forceinline__ void keep_fp32(float& f) { asm("" : "+v"(f)); }
+
 // The raw bits of an io_dtype element (loaded without converting, so a batch of loads stays in flight) and their
 // value.
 template <int IO>
@@ -285,9 +290,11 @@ __global__ __launch_bounds__(kMaxWaves * kWave) void mlstm_multistep_kernel(
 #pragma unroll
               for (int b = 0; b < BV; ++b) {
                 C[j][b] = fmaf(ik, vv[b], fa * C[j][b]);
+                if constexpr (IO == BP_DT_F16 && G == 1) keep_fp32(C[j][b]);
                 hp[g * BV + b] = fmaf(qs, round_io<IO>(C[j][b]), hp[g * BV + b]);
               }
               nn[j] = fmaf(fa, nn[j], ik);
+              if constexpr (IO == BP_DT_F16 && G == 1) keep_fp32(nn[j]);
               qp[g] = fmaf(qs, round_io<IO>(nn[j]), qp[g]);
             }
           }

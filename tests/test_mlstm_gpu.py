@@ -197,6 +197,18 @@ def test_step_equals_multistep_then_lazy_commit(dtype, bv):
         assert torch.equal(a.reshape(-1), b.reshape(-1))
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("bv", [4, 8, 16])
+@pytest.mark.parametrize("nh,dq,dv", [(4, 512, 512), (16, 64, 128)])
+def test_one_position_equals_the_first_of_three(nh, dq, dv, bv, dtype):
+    """A launch of one position (its own instantiation) gives the first position of a launch of three, bit for bit: in
+    float16 too, where a multiply-add and its rounding made one instruction gave a few outputs other bits."""
+    q, k, v, i, f, state = rand_inputs(3, nh, dq, dv, dtype, seed=21)
+    three = run(state, q, k, v, i, f, bv=bv)[0]
+    one = run(state, *(x[:1].contiguous() for x in (q, k, v, i, f)), bv=bv)[0]
+    assert torch.equal(one, three[:1])
+
+
 def test_step_refuses_overlapping_state():
     from byteprof_amd.optim import draft_core as DC
 
