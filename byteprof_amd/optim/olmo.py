@@ -40,7 +40,6 @@ PREFILL_ROWS = 256  # most prompt rows of one pass (its buffers: about 5 (H + F)
 VERIFY_ROWS = 16  # rows of the verify-pass buffers (allocated once per decoder, never reallocated)
 PRO_MAX_ROWS = {"bf16": 3, "int8": 1, "int4": 1}  # most rows of a linear launch with the norm as its prologue
 INT4_PRO_LDS_BYTES = 64 * 1024  # the int4 kernel's norm prologue: rows, gamma, residual rows, gamma2, (2 M + 2) K bf16
-INT4_PRO_MAX_K = INT4_PRO_LDS_BYTES // 8  # widest row it stages at one row
 PRO_LDS_BYTES = 80 * 1024  # the launch keeps gamma and the residual rows in LDS while the staged rows and they fit
 ARGMAX_ROW_WORDS, ARGMAX_ERROR_WORD = 132, 130  # u32 words of the argmax scratch per row; its error word
 
@@ -148,10 +147,8 @@ class OlmoDecoder:
         self.tok, self.pos = z(1, dtype=torch.int64), z(1, dtype=torch.int64)
         self.x, self.xn, self.attn, self.o, self.dn = z(1, H), z(1, H), z(1, H), z(1, H), z(1, H)
         self.h = z(1, H)  # the residual stream after the attention half of a layer (fused-norm step)
-        # the sublayer norms run inside the next linear's launch when its plan keeps whole rows (split 1); the int4
-        # kernel's prologue stages the row, gamma, the residual row and gamma2 in LDS (K <= 8192, bf16 scales)
-        self.fuse_norms = all(self._plan(n, H, 1)[2] == 1 for n in (3 * H, 2 * F, V)) and (
-            kind != "int4" or (H <= INT4_PRO_MAX_K and self.lm_head[1].dtype == torch.bfloat16))
+        # the sublayer norms run inside the next linear's launch when every one of those launches takes the prologue
+        self.fuse_norms = all(self._pro_fits(n, H, 1) for n in (3 * H, 2 * F, V))
         self.qkv, self.gu, self.act, self.logits = z(1, 3 * H), z(1, 2 * F), z(1, F), z(1, V)
         # the argmax's partials, counter and error word: zeroed once, the counter left at zero by every launch
         self.argmax_scratch = z(-(-_lib.lib().bp_decode_argmax_scratch_bytes() // 4), dtype=torch.int32)
@@ -208,7 +205,7 @@ class OlmoDecoder:
                       zero=args[2] if len(args) > 2 else None)
 
     def _step_separate(self) -> None:
-        """The step with a norm launch after o and after down (plans that split K)."""
+        """The step with a norm launch after o and after down (plans that split K, a hidden size of ragged segments)."""
         cfg, L = self.cfg, _lib.lib()
         H, D = cfg.hidden, cfg.head_dim
         st = _lib.stream_ptr(self.device)
@@ -244,20 +241,26 @@ class OlmoDecoder:
             return tile // 16, waves, min(split, k // 128), 0
         return S._resolve(self.kind, n, k, rows, None)
 
+    def _whole_rows(self, n: int, k: int, rows: int) -> bool:
+        """Whether the launch of an n x k linear keeps whole rows of whole segments: no K split, no element loads (int4: the
+        matrix-core kernel, n a multiple of 4). Then it has an epilogue and a prologue."""
+        return self._plan(n, k, rows)[2] == 1 and S.whole_segments(self.kind, k) and (self.kind != "int4" or n % 4 == 0)
+
     def _gate_up_silu(self, x: torch.Tensor, gw: tuple, act: torch.Tensor, gu: torch.Tensor, rows: int) -> None:
         """act[:rows] = bf16(bf16(silu(g)) * u) of the interleaved gate|up projection: one launch with the SiLU
-        product as its epilogue when the shape's K order has no split, else skinny_mm + the SiLU kernel (the same
-        sums either way)."""
+        product as its epilogue when it keeps whole rows, else skinny_mm + the SiLU kernel (the same sums either
+        way)."""
         F, H = self.cfg.ffn, self.cfg.hidden
-        rb, waves, split, xs = self._plan(2 * F, H, rows)
+        rb, waves, _, xs = self._plan(2 * F, H, rows)
+        fuse = rows <= 16 and self._whole_rows(2 * F, H, rows)
         L, st = _lib.lib(), _lib.stream_ptr(self.device)
-        if self.kind == "int4" and split == 1 and rows <= 16 and F % 2 == 0:
+        if self.kind == "int4" and fuse:
             packed, scale, zero = gw
             _lib.check(L.bp_skinny_int4_silu(x.data_ptr(), packed.data_ptr(), scale.data_ptr(),
                                              _lib.TORCH_DT[scale.dtype], zero.data_ptr(), act.data_ptr(), rows, F, H,
                                              16 * rb, waves, st), "bp_skinny_int4_silu")
             return
-        if split == 1 and rows <= 16 and self.kind != "int4":
+        if self.kind != "int4" and fuse:
             sc, sdt = (gw[1].data_ptr(), _lib.TORCH_DT[gw[1].dtype]) if self.kind == "int8" else (None, 0)
             _lib.check(L.bp_skinny_mf_silu(S._KIND_CODE[self.kind], x.data_ptr(), gw[0].data_ptr(), sc, sdt,
                                            act.data_ptr(), rows, F, H, rb, waves, xs, st), "bp_skinny_mf_silu")
@@ -274,8 +277,9 @@ class OlmoDecoder:
         extra = lambda n, k: int(self._plan(n, k, 1)[2] > 1)  # noqa: E731  (the split reduce)
         if self.fuse_norms:
             return 3 + (5 + extra(H, H) + extra(H, F)) * self.cfg.layers
-        # gate|up: the SiLU epilogue in the launch, else the product's own launch after a split's reduce
-        per_layer = 7 + extra(3 * H, H) + extra(H, H) + extra(H, F) + 2 * extra(2 * F, H)
+        # gate|up: the SiLU epilogue in the launch, else the product's own launch (after a split's reduce)
+        silu = int(not self._whole_rows(2 * F, H, 1))
+        per_layer = 7 + extra(3 * H, H) + extra(H, H) + extra(H, F) + extra(2 * F, H) + silu
         return 4 + per_layer * self.cfg.layers + extra(V, H)
 
     def _down_splitk(self, s: int) -> tuple[int, int, int, int] | None:
@@ -310,16 +314,15 @@ class OlmoDecoder:
         self.vws = torch.empty(split * n * H, dtype=torch.float32, device=dev)  # the down launch's partials
 
     def _pro_fits(self, n: int, k: int, rows: int, norms: int = 1) -> bool:
-        """Whether the launch of an n x k linear at rows rows takes a norm prologue: a plan that keeps whole rows
-        (split 1), the rows x k activations staged in LDS (32 KiB), gamma with the residual rows in LDS beside them
+        """Whether the launch of an n x k linear at rows rows takes a norm prologue: a launch that keeps whole rows
+        (_whole_rows), the rows x k activations staged in LDS (32 KiB), gamma with the residual rows in LDS beside them
         (one row, or PRO_LDS_BYTES in all: past it the prologue would read them from memory element by element, which
         made 7-row verify rounds 870 -> 1206 us), and at most PRO_MAX_ROWS rows: measured on the OLMo-2-1B shape
         against the one-round-trip norm launch, the prologue wins at 1..3 rows for bf16 (2 / 3-row rounds 731 / 755
         -> 724 / 749 us; 5 rows loses, 791-808 -> 829 us) and at one row only for int8 (2 / 3 rows: 575 / 586-599
         without it, 587-597 / 631-634 with it) and for int4 (2 / 3 / 5 / 7 rows: 601 / 617 / 642 / 681 us without it,
         619 / 654 / 746 / 867 with it); at one row it saves the norm launch of every sublayer."""
-        _, _, split, _ = self._plan(n, k, rows)
-        if split != 1 or rows > PRO_MAX_ROWS[self.kind]:
+        if rows > PRO_MAX_ROWS[self.kind] or not self._whole_rows(n, k, rows):
             return False
         if self.kind == "int4":  # the int4 kernel's prologue (rows, gamma, residual rows, gamma2 in LDS)
             return (2 * rows + 2) * k * 2 <= INT4_PRO_LDS_BYTES and self.lm_head[1].dtype == torch.bfloat16
@@ -422,7 +425,7 @@ class OlmoDecoder:
                     "qkv": z(n, 3 * H), "act": z(n, F)}
             plans = {(rows, k): self._plan(rows, k, 1)[1:3] for rows, k in ((3 * H, H), (H, H), (2 * F, H), (H, F))}
             need = max((split * n * rows for (rows, _), (_, split) in plans.items() if split > 1), default=0)
-            if plans[(2 * F, H)][1] > 1:  # a split gate|up has no SiLU epilogue
+            if not self._whole_rows(2 * F, H, 1):  # gate|up without the SiLU epilogue
                 bufs["gu"] = z(n, 2 * F)
             bufs["ws"] = z(max(1, need), dtype=torch.float32)
             self._prefill, self._prefill_plans = bufs, plans

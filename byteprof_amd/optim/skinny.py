@@ -72,6 +72,12 @@ def k_segment(kind: str) -> int:
     return 64 if kind == "bf16" else 128
 
 
+def whole_segments(kind: str, k: int) -> bool:
+    """Whether a bf16 / int8 launch over K loads whole segments (on 16-byte aligned operands; int4's K is whole groups).
+    Only such launches have the SiLU epilogue and the norm prologues: other K take the element loads, plain products."""
+    return kind == "int4" or (k % k_segment(kind) == 0 and k < 1 << 24)
+
+
 def _default_waves(kind: str, n: int, k: int) -> int:
     """Waves sharing K: 4 from 2 segments a wave on (1280 x 4736 bf16 at one row: 5.1 us with 4, 5.7 with 8); 8 for
     int8 weights of few rows and a long K, whose 9..64-row launches have too few waves otherwise (1280 x 4736 at 16

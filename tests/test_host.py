@@ -5,6 +5,7 @@ tests/test_skinny.py:125-132."""
 
 from __future__ import annotations
 
+import ctypes
 import json
 from pathlib import Path
 
@@ -13,6 +14,7 @@ import pytest
 import torch
 import torch.nn as nn
 
+from byteprof_amd import _lib
 from byteprof_amd.optim import skinny as S
 from byteprof_amd.quant import accounting as A
 from byteprof_amd.quant import select as SEL
@@ -471,3 +473,26 @@ def test_every_mutant_plants_its_text_once():
         if new is None:
             continue
         assert (pkg / rel).read_text().count(old) == 1, name
+
+
+@pytest.mark.parametrize("kind,k", [("bf16", 224), ("bf16", 200), ("bf16", 480), ("int8", 448), ("int8", 576),
+                                    ("int8", 64)])
+def test_decoders_fuse_only_launches_that_the_library_takes(kind, k):
+    """A hidden size that is not whole segments of the kind: the library refuses its prologue and SiLU launches (before
+    anything runs), so the decoder must not plan them, whatever the plan's split."""
+    from byteprof_amd.optim import olmo as OG
+    L, code = _lib.lib(), S._KIND_CODE[kind]
+    pro = S.BpPrologue(S.PRO_NORM, 1e-6, 0x1000, 0x2000, None, None)
+    assert not S.whole_segments(kind, k) and S.whole_segments(kind, 4 * S.k_segment(kind))
+    dec = OG.OlmoDecoder.__new__(OG.OlmoDecoder)
+    dec.kind = kind
+    for n in (512, 3 * k, 5000, 100352):
+        assert L.bp_skinny_mf_pro(code, 0x10000, 0x20000, 0x30000, 1, 0x40000, 1, n, k, 1, 4, 0, ctypes.byref(pro),
+                                  None) == _lib.BP_E_UNSUPPORTED
+        assert L.bp_skinny_mf_silu(code, 0x10000, 0x20000, 0x30000, 1, 0x40000, 1, n, k, 1, 4, 0,
+                                   None) == _lib.BP_E_UNSUPPORTED
+        for rows in (1, 2, 3, 16):
+            assert not dec._pro_fits(n, k, rows) and not dec._whole_rows(n, k, rows)
+        dec.kind = "int4"  # the int4 matrix-core kernel: groups of four weight rows
+        assert dec._whole_rows(512, 256, 1) and not dec._whole_rows(1001, 256, 1)
+        dec.kind = kind

@@ -330,6 +330,41 @@ def _deq4(args) -> np.ndarray:
                               zero.float().cpu().numpy()).astype(np.float32)
 
 
+# hidden sizes that are not whole segments (64 bf16 or 128 int8 elements), and an int4 vocabulary off the groups of four
+RAGGED = {"h224": OG.OlmoConfig(hidden=224, ffn=512, layers=2, heads=7, vocab=512, max_len=96),
+          "h448": OG.OlmoConfig(hidden=448, ffn=896, layers=2, heads=7, vocab=512, max_len=96),
+          "v1001": OG.OlmoConfig(hidden=128, ffn=256, layers=2, heads=2, vocab=1001, max_len=96)}
+
+
+@pytest.mark.parametrize("kind,shape", [("bf16", "h224"), ("bf16", "h448"), ("int8", "h224"), ("int8", "h448"),
+                                        ("int4", "v1001")])
+def test_ragged_decoders_match_the_oracle(kind, shape):
+    """Decoders whose linears take the element loads (no epilogue, no prologue) or the int4 VALU kernel: the steps against
+    the oracle, the prompt passes against the steps, and a verify pass against the steps."""
+    cfg = RAGGED[shape]
+    dec, W, oc = _small_decoder(kind, cfg=cfg)
+    assert dec.fuse_norms == all(dec._whole_rows(n, cfg.hidden, 1) for n in (3 * cfg.hidden, 2 * cfg.ffn, cfg.vocab))
+    prompt = [3, 17, 99, 250, 7] * 8
+    toks, logits = OO.greedy(W, oc, prompt, 4)
+    dec.pos.zero_()
+    steps = []
+    for t in prompt + toks[:-1]:
+        dec.tok.fill_(t)
+        dec.step()
+        steps.append(dec.logits.clone())
+    for got, want in zip(steps[len(prompt) - 1:], logits):
+        assert ON.normwise_error(_np(got[0]), want) < GATE
+    dec.prefill(torch.tensor(prompt))
+    assert torch.equal(dec.logits, steps[len(prompt) - 1]) and int(dec.pos) == len(prompt)
+    dec.verify_buffers(8)
+    for s in (1, 3, 8):  # the rows of a verify pass over the prompt's last tokens: the steps at their positions
+        dec.v_ids[:s].copy_(torch.tensor(prompt[-s:]))
+        dec.v_pos.fill_(len(prompt) - s)
+        dec.verify(s)
+        want = torch.cat(steps[len(prompt) - s:len(prompt)])
+        assert torch.equal(dec.vlogits[:s], want), s
+
+
 @pytest.mark.parametrize("shape", ["small", "fused"])
 @pytest.mark.parametrize("kind", ["bf16", "int8", "int4"])
 def test_decode_steps_match_the_oracle(kind, shape):
