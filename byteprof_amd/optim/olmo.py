@@ -415,8 +415,10 @@ class OlmoDecoder:
         c(L.bp_draft_verify_next(self.v_ids.data_ptr(), self.v_tok.data_ptr(), self.v_out.data_ptr(),
                                  self.v_pos.data_ptr(), s, self.smax, st), "bp_draft_verify_next")
 
+    @torch.inference_mode(False)
     def _prefill_buffers(self) -> dict[str, torch.Tensor]:
-        """The buffers of prompt passes (allocated at the first prompt of more than one token and kept)."""
+        """The buffers of prompt passes (allocated at the first prompt of more than one token and kept: ordinary tensors, so
+        that a prompt inside torch.inference_mode may come first and one outside it later)."""
         bufs = getattr(self, "_prefill", None)
         if bufs is None:
             H, F, n = self.cfg.hidden, self.cfg.ffn, PREFILL_ROWS

@@ -36,3 +36,16 @@ def test_prefill_equals_the_one_token_steps(kind, shape, monkeypatch):
         for name, a, b in zip(("k", "v", "logits", "tok", "pos"), got, want):
             assert torch.equal(a, b), (length, name)
         assert torch.isfinite(dec.logits.float()).all() and int(dec.pos) == length
+
+
+def test_prompts_inside_and_outside_inference_mode():
+    """The pass buffers are made at the first prompt: one inside torch.inference_mode, then one outside it, and a
+    generate() each way, give the same tokens."""
+    cfg = CFGS["odd"]
+    dec = OG.OlmoDecoder(cfg, OG.random_weights(cfg, DEV, seed=5), "bf16")
+    gen = OG.make_generate(dec)
+    prompt = torch.tensor([[5, 9, 2, 700, 31]])
+    with torch.inference_mode():
+        inside = gen(prompt, max_new_tokens=4)
+    outside = gen(prompt, max_new_tokens=4)
+    assert torch.equal(inside.cpu(), outside.cpu())
