@@ -766,7 +766,7 @@ __global__ __launch_bounds__(kBlock) void norm_residual_kernel(const uint16_t* _
                                                                const uint16_t* __restrict__ w,
                                                                const uint16_t* residual, uint16_t* out, int n,
                                                                float eps) {
-  extern __shared__ uint16_t norm_xs[];
+  extern __shared__ __align__(16) uint16_t norm_xs[];
   const int64_t row = static_cast<int64_t>(blockIdx.x) * n;
   for (int i = threadIdx.x; i < n; i += blockDim.x) norm_xs[i] = x[row + i];
   __syncthreads();
@@ -786,7 +786,7 @@ __global__ __launch_bounds__(kNormVecThreads) void norm_residual_vec_kernel(cons
                                                                             const uint16_t* __restrict__ w,
                                                                             const uint16_t* residual, uint16_t* out,
                                                                             int n, float eps) {
-  extern __shared__ uint16_t norm_xs[];
+  extern __shared__ __align__(16) uint16_t norm_xs[];
   const int64_t row = static_cast<int64_t>(blockIdx.x) * n;
   const int pieces = n / 8;
   const bool res = residual != nullptr;
@@ -838,7 +838,7 @@ __global__ __launch_bounds__(kBlock) void splitk_norm_residual_kernel(const floa
                                                                       const uint16_t* __restrict__ w,
                                                                       const uint16_t* residual, uint16_t* out, int n,
                                                                       float eps) {
-  extern __shared__ uint16_t norm_xs[];
+  extern __shared__ __align__(16) uint16_t norm_xs[];
   const int64_t total = static_cast<int64_t>(gridDim.x) * n;
   const int64_t row = static_cast<int64_t>(blockIdx.x) * n;
   for (int i = threadIdx.x; i < n; i += blockDim.x) {

@@ -403,7 +403,7 @@ __device__ __forceinline__ void mf_fold_halves(floatx4 (&acc)[RB][MB]) {
 
 // LDS image of the folded wave tiles: red[wave][rb][b][q][t], q = m + 8 (row / 4), t = row % 4.
 template <int WAVES, int RB, int MB>
-struct MfRed {
+struct alignas(16) MfRed {  // written in 16-byte pieces
   float v[WAVES][RB][MB][16][4];
 };
 

@@ -28,10 +28,12 @@ __global__ __launch_bounds__(WAVES* kWave, 2) void skinny_wide_kernel(const uint
   constexpr int D = wide_depth<KIND, MB, RP>();
   constexpr int NT = WAVES * kWave;
   constexpr uint32_t kPast = 0x80000000u;  // beyond any resource
-  __shared__ union {
+  union alignas(16) Shared {  // both are read and written in 16-byte pieces
     float red[WAVES][MB][kWave][4];
     uint8_t patch[WAVES][2][2048 * P];
-  } sh;
+  };
+  static_assert(alignof(Shared) == 16 && sizeof(Shared::patch[0][0]) % 16 == 0, "16-byte LDS operations");
+  __shared__ Shared sh;
   __shared__ __align__(16) float row_scale[KIND == kInt8 ? 16 * RP : 1];
 
   const int lane = threadIdx.x & (kWave - 1);
