@@ -89,9 +89,13 @@ __device__ __forceinline__ u32x4 mf_load_w16(const uint8_t* __restrict__ wrow, i
       for (int e = 0; e < 8; ++e)
         if (k + e < K) d[e >> 1] |= static_cast<uint32_t>(p[k + e]) << (16 * (e & 1));
     } else {
+      // against the bytes left, not against K: 68 scalar registers a wave at up to 8 rows instead of 96, so 8 waves a SIMD
+      // run and not 7 (16384 x 8190 at one row 246 us with 96, 163 with 68; small launches lose a little, 300 x 1000 5.9
+      // and 6.4)
+      const int64_t left = K - k;
 #pragma unroll
       for (int e = 0; e < 16; ++e)
-        if (k + e < K) d[e >> 2] |= static_cast<uint32_t>(wrow[k + e]) << (8 * (e & 3));
+        if (e < left) d[e >> 2] |= static_cast<uint32_t>(wrow[k + e]) << (8 * (e & 3));
     }
     return u32x4{d[0], d[1], d[2], d[3]};
   }
