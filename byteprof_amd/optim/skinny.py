@@ -100,10 +100,21 @@ def _default_rb(kind: str, n: int, bucket: int) -> int:
 
 def _default_split(kind: str, n: int, k: int, waves: int) -> int:
     """K ranges in separate workgroups: only for a K so long that a wave's share outweighs the reduce launch (about
-    2.5 us: 1920 x 7168 bf16 at one row takes 6.8 us without a split, 9.1 with 2; 300 x 1024 2.6 and 4.4)."""
+    2.5 us: 1920 x 7168 bf16 at one row takes 6.8 us without a split, 9.1 with 2; 300 x 1024 2.6 and 4.4).
+
+    A K off the segments takes the element loads (4 waves, one segment in flight), where a segment costs a wave 1 to 2 us:
+    past eight segments a wave the split grows while a wave keeps two (four past 8 ranges: the reduce reads every range)
+    and the card has room, 1024 workgroups. us at one row without a split / with the rule's, one MI355X: bf16 512 x 8191
+    86 / 16 (8 ranges), 64 x 8190 53 / 12 (8), 1025 x 2049 22 / 9.0 (8), 4100 x 2050 24 / 19 (2). Below that a split gains
+    less on the device (int8 1025 x 2049 at 5 rows 16.4 / 11.2) than its workspace and second launch cost an eager call's
+    host (21.8 us a call without, 24.7 with)."""
     blocks = -(-n // 8)
     nseg = -(-k // k_segment(kind))
     split = 1
+    if not whole_segments(kind, k):
+        while nseg > 32 and blocks * split < 1024 and nseg > 8 * split * (1 if split < 8 else 2):
+            split *= 2
+        return split
     while blocks * split < 256 and nseg // (waves * split * 2) >= 64:
         split *= 2
     return split

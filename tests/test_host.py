@@ -496,3 +496,18 @@ def test_decoders_fuse_only_launches_that_the_library_takes(kind, k):
         dec.kind = "int4"  # the int4 matrix-core kernel: groups of four weight rows
         assert dec._whole_rows(512, 256, 1) and not dec._whole_rows(1001, 256, 1)
         dec.kind = kind
+
+
+@pytest.mark.parametrize("kind,n,k", [("bf16", 512, 8191), ("bf16", 64, 8190), ("bf16", 1025, 2049), ("int8", 512, 8191),
+                                      ("int8", 8, 30001), ("int8", 1025, 4100)])
+def test_default_plans_split_a_long_ragged_k(kind, n, k):
+    """A K off the segments runs the element loads, one segment at a time: with few weight rows the default plan leaves a
+    wave no more than eight of them in series, at every row count the same order, and splits nothing for a short K or
+    for weight rows that fill the card."""
+    orders = {S._resolve(kind, n, k, m, None)[1:3] for m in (1, 5, 9, 16, 33, 64)}
+    assert len(orders) == 1
+    split = orders.pop()[1]
+    nseg = -(-k // S.k_segment(kind))
+    assert 1 < split <= nseg and nseg / (4 * split) <= 8
+    assert S._default_split(kind, n, 7 * S.k_segment(kind) + 1, 4) == 1
+    assert S._default_split(kind, 16384, k, 4) == 1
