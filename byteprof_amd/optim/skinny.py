@@ -78,29 +78,60 @@ def whole_segments(kind: str, k: int) -> bool:
     return kind == "int4" or (k % k_segment(kind) == 0 and k < 1 << 24)
 
 
+# The default plans: us on one MI355X, weights from memory, one launch of a captured graph.
+
+
 def _default_waves(kind: str, n: int, k: int) -> int:
-    """Waves sharing K: 4 from 2 segments a wave on (1280 x 4736 bf16 at one row: 5.1 us with 4, 5.7 with 8); 8 for
-    int8 weights of few rows and a long K, whose 9..64-row launches have too few waves otherwise (1280 x 4736 at 16
-    rows: 7.4 us with 8, 8.7 with 4; at one row 4.8 and 4.6)."""
+    """Waves sharing K (one K order for every row count).
+
+    bf16: 8 from 96 segments on, 4 from 8 on, 2 from 4 on (4096 x 32768 at one row 54.9 with 4, 48.4 with 8; 1280 x 4736
+    4.9 and 5.3; 300 x 1024 2.6 and 3.4). From 2048 weight rows on the card is full without the last halving of a short K:
+    4 from 12 segments on, 2 from 8 on (32000 x 512 at one row 8.8 with 4, 7.6 with 2; 2048 x 256 2.6 with 2, 2.4 with 1;
+    past 8 rows the wide kernel pays for it: 2048 x 256 at 16 rows 2.8 and 3.3).
+    int8: 8 for a long K under 4096 weight rows, whose 9..64-row launches have too few waves otherwise (1280 x 4736 at 16
+    rows 7.4 with 8, 8.7 with 4; at one row 4.8 and 4.6), else 4 from 8 segments on, but 2 at just 8 from 10240 rows on
+    (32000 x 1024 at one row 10.3 with 4, 8.4 with 2)."""
     nseg = -(-k // k_segment(kind))
-    if kind == "int8" and nseg >= 32 and n < 4096:
-        return 8
-    return 4 if nseg >= 8 else 2 if nseg >= 4 else 1
+    if kind == "int8":
+        if nseg >= 32 and n < 4096:
+            return 8
+        return 4 if nseg >= (9 if n >= 10240 else 8) else 2 if nseg >= 4 else 1
+    full = n >= 2048
+    return 8 if nseg >= 96 else 4 if nseg >= (12 if full else 8) else 2 if nseg >= (8 if full else 4) else 1
 
 
-def _default_rb(kind: str, n: int, bucket: int) -> int:
-    """8-row weight blocks per workgroup: 1 while that leaves no more than two workgroups per CU, else 4 (each
-    activation operand then serves 32 weight rows: 5000 x 6016 bf16 at 8 rows 21.5 us with 1, 16.8 with 4; int8 at one
-    row 10.1 and 9.2), but 1 for bf16 at one row (16000 x 1984: 12.0 us with 1, 12.3 with 4). Past 8 rows the launch
-    picks its own tile."""
-    if n < 4096 or bucket > 8 or (kind == "bf16" and bucket == 1):
+def _default_rb(kind: str, n: int, k: int, m: int) -> int:
+    """8-row weight blocks per workgroup at m rows: each activation operand serves 8 times as many weight rows, but there
+    are as many fewer workgroups. Past 8 rows the launch picks its own tile.
+
+    Up to 2560 weight rows 1 (2048 x 4096 bf16 at 5 rows 5.2, with two 6.4). int8: 2 (4096 x 8192 at one row 8.9, 9.3 with
+    one and 12.8 with four; 16000 x 4096 at 5 rows 15.4, 17.4, 16.6), 4 at 6..8 rows of 4608 to 8192 (8192 x 14336 at 8 rows
+    40 with one, 27.5, 25.2) and for a short K (8192 x 1024 at one row 6.1 with one, 4.8, 4.5), but from 10240 rows on there
+    too 2 past 4 segments. bf16, whose activation operands are half as long: 1 up to 5 rows (16000 x 8192 at 5 rows 45, 48
+    with two, 55), then 4 for 4608 to 8191 rows (6144 x 3072 at 8 rows 10.9 with one, 9.3) and 2 past them (32000 x 4096 at
+    8 rows 51 with one, 45); a short K 2 (32000 x 512 at 5 rows 7.9 with one, 7.6)."""
+    if n < 2560 or m > 8:
         return 1
-    return 4
+    nseg = -(-k // k_segment(kind))
+    short = nseg <= 8
+    if kind == "int8":
+        if short and n >= 4608:
+            return 4 if nseg <= 4 or n < 10240 else 2
+        return 4 if m > 5 and 4608 <= n <= 8192 else 2
+    if short:
+        return 2 if m > 5 or n >= 4608 else 1
+    if m <= 5 or n < 4608:
+        return 1
+    return 4 if n < 8192 else 2
 
 
 def _default_split(kind: str, n: int, k: int, waves: int) -> int:
-    """K ranges in separate workgroups: only for a K so long that a wave's share outweighs the reduce launch (about
-    2.5 us: 1920 x 7168 bf16 at one row takes 6.8 us without a split, 9.1 with 2; 300 x 1024 2.6 and 4.4).
+    """K ranges in separate workgroups: a second launch (the reduce, about 2.5 us) and a workspace, so only for a long K
+    over few weight rows: from 160 segments (int8: 112) on, while a wave keeps four and the first launch has fewer than
+    192 workgroups (bf16 at 16 rows without / with: 64 x 32768 36 / 10.6 (8 ranges), 300 x 14336 19 / 9.7 (4); int8 64 x
+    32768 26 / 9.9; at one row 13.3 / 6.9, 7.9 / 6.3, 10.9 / 6.7), and for bf16 at 32 segments a wave up to 512 (2048 x
+    32768 at one row 26.7 / 27.4, at 16 rows 43 / 30). Below that the plain launch is the faster one up to 8 rows (512 x 8192 bf16
+    5.1 and 5.6; 1920 x 7168 6.8 and 9.1; 300 x 1024 2.6 and 4.4), though not at 16 (512 x 8192 11.2 and 8.1).
 
     A K off the segments takes the element loads (4 waves, one segment in flight), where a segment costs a wave 1 to 2 us:
     past eight segments a wave the split grows while a wave keeps two (four past 8 ranges: the reduce reads every range)
@@ -115,8 +146,10 @@ def _default_split(kind: str, n: int, k: int, waves: int) -> int:
         while nseg > 32 and blocks * split < 1024 and nseg > 8 * split * (1 if split < 8 else 2):
             split *= 2
         return split
-    while blocks * split < 256 and nseg // (waves * split * 2) >= 64:
-        split *= 2
+    if nseg >= (112 if kind == "int8" else 160):
+        while (spw := nseg // (waves * split)) >= 8 and (
+                blocks * split < 192 or (kind == "bf16" and spw >= 32 and blocks * split <= 512)):
+            split *= 2
     return split
 
 
@@ -133,13 +166,13 @@ def _table_plan(kind: str, n: int, k: int, m: int, pro: bool = False) -> tuple[i
     bucket = _bucket(m)
     entry = _TABLE.get((kind, n, k))
     if entry is not None:
-        rb = int(entry.get("rb", {}).get(str(bucket), _default_rb(kind, n, bucket)))
+        rb = int(entry.get("rb", {}).get(str(bucket), _default_rb(kind, n, k, m)))
         if pro:
             rb = int(entry.get("rb_pro", {}).get(str(bucket), rb))
         xs = int(entry.get("xs", {}).get(str(bucket), 0))
         return rb, int(entry["waves"]), int(entry.get("split", 1)), xs
     waves = _default_waves(kind, n, k)
-    return _default_rb(kind, n, bucket), waves, _default_split(kind, n, k, waves), 0
+    return _default_rb(kind, n, k, m), waves, _default_split(kind, n, k, waves), 0
 
 
 def _resolve(kind: str, n: int, k: int, m: int, cfg, pro: bool = False) -> tuple[int, int, int, int]:

@@ -511,3 +511,27 @@ def test_default_plans_split_a_long_ragged_k(kind, n, k):
     assert 1 < split <= nseg and nseg / (4 * split) <= 8
     assert S._default_split(kind, n, 7 * S.k_segment(kind) + 1, 4) == 1
     assert S._default_split(kind, 16384, k, 4) == 1
+
+
+def test_default_plans_over_the_range():
+    """Outside the table: one K order for every row count, compiled for every launch form (plain and with a prologue), no
+    wave without a segment, K split only where the first launch leaves the card idle, and at few rows no fewer workgroups
+    than CUs where the weight rows allow 256."""
+    ns = (1, 8, 64, 300, 1024, 2047, 2048, 2560, 3072, 4096, 4608, 5000, 8192, 10240, 16000, 32000)
+    for kind in ("bf16", "int8"):
+        seg = S.k_segment(kind)
+        for n in ns:
+            for nseg in (1, 2, 3, 4, 5, 7, 8, 9, 11, 12, 31, 32, 64, 95, 96, 111, 112, 159, 160, 224, 512):
+                k = nseg * seg
+                if (kind, n, k) in S._TABLE:
+                    continue
+                plans = {m: S._resolve(kind, n, k, m, None) for m in (1, 2, 5, 6, 8, 9, 16, 17, 32, 33, 64)}
+                assert len({p[1:3] for p in plans.values()}) == 1, (kind, n, k, plans)
+                rb, waves, split, xs = plans[1]
+                assert xs == 0 and waves * split <= nseg or (waves, split) == (1, 1), (kind, n, k, plans[1])
+                blocks = -(-n // 8)
+                assert split == 1 or (nseg >= 112 and blocks <= 512 and nseg // (waves * split) >= 4)
+                for m, p in plans.items():
+                    assert p[0] == 1 or (m <= 8 and blocks // p[0] >= 144), (kind, n, k, m, p)
+                    if m <= 3 and split == 1 and S._stage_bytes(kind, m, k, 1) >= 0:
+                        assert S._resolve(kind, n, k, m, None, pro=True)[1:3] == p[1:3]
