@@ -112,7 +112,7 @@ int skinny_int4_launch(const void* x, const void* packed, const void* scale, int
   if ((epi != 0 || pro.kind != 0) && !mf) return BP_E_UNSUPPORTED;
   const int64_t tiles = tile_rows > 0 ? (N + tile_rows - 1) / tile_rows : 0;
   if (tiles > 0x7fffffff) return BP_E_INVALID_ARG;
-  const int nb = mf && pro.kind == 0 ? int4_wide_nb(M, K, tiles) : 0;
+  const int nb = mf && pro.kind == 0 && waves > 0 ? int4_wide_nb(M, K, tiles, tile_rows, waves, split) : 0;
   if (nb == 0 && M > 16) {  // the VALU kernel: 16 rows a launch
     for (int64_t r = 0; r < M; r += 16) {
       const int rc = skinny_int4_launch(static_cast<const uint16_t*>(x) + r * K, packed, scale, scale_dt, zero,

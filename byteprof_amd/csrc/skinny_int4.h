@@ -11,14 +11,19 @@ using Int4WideFn = void (*)(const uint16_t*, const uint8_t*, const void*, const 
                             int64_t, int);
 Int4WideFn int4_wide_pick(int nb, int tile_rows, int waves, int scale_dt, int epi);
 
-// Activation blocks per workgroup of a launch, or 0 where skinny_int4.hip's kernel runs it (the same bits). A few rows of
-// few tiles are its: its waves have more groups in flight (one row of 2048 x 8192 in 128 tiles 6.6 us, wide 8.6; five
-// rows 7.8 and 8.7, nine 9.0 and 8.8; but 2048 x 2048 five rows 4.3 and 4.0, and in 256 tiles 8192 x 2048 one row 5.3 and
-// 4.8). Two blocks per workgroup read the codes once for 32 rows and take about 1.8 times one block's time: by the
-// rounds of workgroups over 256 CUs (8192 x 2048 at 33 rows, three blocks: one 8.7 us, two 10.4; at 20 rows 7.4 and 6.7).
-inline int int4_wide_nb(int64_t M, int64_t K, int64_t tiles) {
+// Activation blocks per workgroup of a launch, or 0 where skinny_int4.hip's kernel runs it (the same bits). A few rows of a
+// long K in 16-row tiles are its: its waves have four groups in flight, the wide kernel's two. us on one MI355X, that
+// kernel / the wide one, by the groups a wave walks (any number of tiles): 4 groups (2048 x 2048 in 128 tiles) one row 4.1
+// / 4.3, two 4.3 / 4.3, four 4.7 / 4.4; 8 groups (4096 x 4096 in 256) one row 5.3 / 6.1, five 5.8 / 6.1, eight 6.7 / 6.1;
+// 16 (2048 x 8192) one row 7.0 / 9.0, five 7.7 / 9.0, eight 9.3 / 9.0; 2 groups (4096 x 1024) 4.0 / 3.6. In tiles of 32
+// and 64 rows the wide kernel is the faster at one row already (6144 x 4096 7.9 / 6.7, 64000 x 2048 19.3 / 18.0; 8192 x
+// 8192 11.7 / 11.9). Two blocks per workgroup read the codes once for 32 rows and take about 1.8 times one block's time:
+// by the rounds of workgroups over 256 CUs (8192 x 2048 at 33 rows, three blocks: one 8.7 us, two 10.4; at 20 rows 7.4
+// and 6.7).
+inline int int4_wide_nb(int64_t M, int64_t K, int64_t tiles, int tile_rows, int waves, int split) {
+  const int64_t per_wave = K / 128 / (static_cast<int64_t>(waves) * split);
+  if (tile_rows == 16 && ((M < 8 && per_wave >= 8) || (M <= 2 && per_wave >= 4))) return 0;
   const int64_t blocks = (M + 15) / 16;
-  if (M <= 8 && tiles < 256 && (M <= 4 || K >= 4096)) return 0;
   if (blocks == 1) return 1;
   const int64_t one = (tiles * blocks + 255) / 256, two = (tiles * ((blocks + 1) / 2) + 255) / 256;
   return 10 * one <= 18 * two ? 1 : 2;

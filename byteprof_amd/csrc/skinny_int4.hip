@@ -459,14 +459,15 @@ Int4MfFn int4_mf_dtype(int waves, int scale_dt) {
   }
 }
 
+// Tiles of 32 and 64 rows only with a prologue: without one skinny_int4_wide.hip runs them (int4_wide_nb).
 template <int EPI, bool PRO>
 Int4MfFn int4_mf_tile(int tile_rows, int waves, int scale_dt) {
-  switch (tile_rows) {
-    case 16: return int4_mf_dtype<1, 4, EPI, PRO>(waves, scale_dt);
-    case 32: return int4_mf_dtype<2, 3, EPI, PRO>(waves, scale_dt);
-    case 64: return int4_mf_dtype<4, 2, EPI, PRO>(waves, scale_dt);
-    default: return nullptr;
+  if (tile_rows == 16) return int4_mf_dtype<1, 4, EPI, PRO>(waves, scale_dt);
+  if constexpr (PRO) {
+    if (tile_rows == 32) return int4_mf_dtype<2, 3, EPI, PRO>(waves, scale_dt);
+    if (tile_rows == 64) return int4_mf_dtype<4, 2, EPI, PRO>(waves, scale_dt);
   }
+  return nullptr;
 }
 
 template <int MT, int RB>

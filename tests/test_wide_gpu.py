@@ -83,18 +83,19 @@ def test_the_rule_takes_every_tile_it_may_pick():
 @pytest.mark.parametrize("tile_rows", [16, 32, 64])
 @pytest.mark.parametrize("n,groups,waves,split,sdt", [(4, 1, 4, 1, None), (68, 3, 2, 1, torch.float16),
                                                       (300, 9, 8, 2, torch.float32), (1000, 32, 1, 1, None),
-                                                      (17000, 2, 4, 1, None)])
+                                                      (17000, 2, 4, 1, None), (132, 16, 4, 1, torch.float16),
+                                                      (132, 64, 4, 2, None)])
 def test_int4_rows_equal_the_one_row_launch(tile_rows, n, groups, waves, split, sdt):
     """bp_skinny_int4_rows at 1..64 rows (one and two activation blocks per workgroup, one and several activation tiles,
-    partial weight tiles, waves without a group): each row equal bit for bit to its own launch, which with these few tiles
-    is the 16-row kernel's (17000 rows: the wide one's)."""
+    partial weight tiles, waves without a group): each row equal bit for bit to its own launch. In 16-row tiles the 16-row
+    kernel takes the one-row launch from 4 groups a wave on, and up to 7 rows from 8 groups on: both sides of those lines."""
     k = groups * S.GROUP
     w = (torch.randn(n, k, generator=torch.Generator(device=DEV).manual_seed(n), device=DEV) * 0.02).to(torch.bfloat16)
     packed, scale, zero = S.quantize_int4(w, tile_rows)
     scale = scale if sdt is None else scale.to(sdt)
     x = randn_x(64, k, seed=n)
     ones = torch.cat([S.skinny_mm(x[r:r + 1].contiguous(), packed, scale, zero, cfg=(waves, split)) for r in range(64)])
-    for m in (5, 9, 16, 17, 32, 33, 49, 64):
+    for m in (2, 3, 5, 7, 8, 9, 16, 17, 32, 33, 49, 64):
         got = S.skinny_mm(x[:m].contiguous(), packed, scale, zero, cfg=(waves, split))
         assert torch.equal(got.view(torch.int16), ones[:m].view(torch.int16)), m
     check_against_oracle(got, x, S.dequantize("int4", packed, scale, zero).cpu().numpy())
