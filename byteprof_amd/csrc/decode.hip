@@ -80,15 +80,17 @@ constexpr int kAttnWaves = kAttnThreads / kWave;
 // are packed (v_dot2_f32_bf16, two of them an operation), a round's reductions share their steps, and S workgroups share
 // a head: each reads the head's whole K rows for the scores (they run on one XCD and meet in its L2), and only its own
 // columns of V. Launches of many rows have workgroups enough (S = 1). The order of every sum is the same for every S:
-//   - scores: LPR lanes per cache row (16 bytes each, whole lines), four row batches per round and the next round's loads
-//     in flight; a lane's 8 products by v_dot2_f32_bf16 in order, then a butterfly over the row's lanes (distances LPR/2
+//   - scores: LPR lanes per cache row (16 bytes each, whole lines), four row batches per round; a lane's 8 products by v_dot2_f32_bf16 in order, then a butterfly over the row's lanes (distances LPR/2
 //     .. 1) for the round's rows at once. s_t = bf16(bf16(q . k_t) * scale), p = bf16(softmax_fp32(s));
 //   - values: position t belongs to class t % C (C = 512 SMAX / LPR). A thread adds its class's positions in order, two
 //     at a time (t and t + C: v_dot2_f32_bf16 on the pair); the classes are added as a tree over the bits of the class:
 //     the highest first (with S = 1 the two classes a thread holds, else a lane bit), then the lowest on, lanes by
 //     butterflies, then waves through LDS.
-// A row can be taken from LDS instead of the cache (SUB: the rows the launch itself writes). RING: the rounds of K rows
-// whose registers a thread holds (1: a launch of many workgroups hides the latency with them, at 64 registers a thread).
+// A row can be taken from LDS instead of the cache (SUB: the rows the launch itself writes).
+// One round of loads is in flight, and a round's four scores are computed without branches: a second round's copies of the
+// loops cost short contexts more code to fetch than long ones gained (us a launch, 16 heads of 128, with a second round
+// and a branch per batch / without: one row at 5 positions 4.5 / 4.3, 108 4.7 / 4.4, 1900 16.2 / 14.0; 9 rows at 64 7.1 /
+// 6.9, 1000 14.2 / 13.5).
 template <int LPR>
 struct AttnShape {
   static constexpr int D = 8 * LPR;
@@ -107,7 +109,7 @@ __device__ __forceinline__ void reduce_rows(float* v, int lane, int& first) {
   }
 }
 
-template <int LPR, int S, bool SUB, int RING>
+template <int LPR, int S, bool SUB>
 struct HeadAttention {
   using A = AttnShape<LPR>;
   static constexpr int D = A::D, C = A::C;
@@ -115,7 +117,6 @@ struct HeadAttention {
   static constexpr int STEP = kAttnWaves * RPW;       // K rows per workgroup-wide batch
   static constexpr int KU = 4;                        // batches per round
   static constexpr int LV = LPR / S;                  // lanes per value row
-  static constexpr int VSTEP = kAttnThreads / LV;     // value rows per workgroup-wide batch
   static constexpr int NU = A::SMAX / S;              // classes a thread holds
   static constexpr int VB = 2 / NU;                   // pairs of C rows per round
   static constexpr int VU = 2 * NU * VB;              // batches per round
@@ -176,10 +177,8 @@ struct HeadAttention {
     float dot[KU];
 #pragma unroll
     for (int u = 0; u < KU; ++u) {
-      const int b0 = t0 + u * STEP;  // the batch's first row: the branches are the workgroup's
-      dot[u] = 0.f;
-      if (b0 >= T) continue;
-      u32x4 w = kv[u];
+      const int b0 = t0 + u * STEP;  // the batch's first row
+      u32x4 w = kv[u];  // zeros past the end
       if constexpr (SUB) {
         const int t = b0 + slot;
         if (b0 + STEP > sub_lo && t >= sub_lo && t < T)
@@ -240,35 +239,11 @@ struct HeadAttention {
     const u32x4 q = *reinterpret_cast<const u32x4*>(qs + 8 * s);
     float m = -INFINITY;
     constexpr int R = KU * STEP;
-    if constexpr (RING == 1) {
-      scores(k0, 0, q, ksub, sub_lo, scale, sc, m);
-      for (int t0 = R; t0 < T; t0 += R) {
-        load_k(t0, k0);
-        scores(k0, t0, q, ksub, sub_lo, scale, sc, m);
-      }
-    } else {
-      // often few positions: the next round's loads only where there is one (a load past the end costs
-      // the address unit's time), each case on its own path, so that the waits stay exact
-      u32x4 k1[KU];
-      for (int t0 = 0;; t0 += 2 * R) {
-        if (t0 + R >= T) {
-          scores(k0, t0, q, ksub, sub_lo, scale, sc, m);
-          break;
-        }
-        load_k(t0 + R, k1);
-        scores(k0, t0, q, ksub, sub_lo, scale, sc, m);
-        if (t0 + 2 * R >= T) {
-          scores(k1, t0 + R, q, ksub, sub_lo, scale, sc, m);
-          break;
-        }
-        load_k(t0 + 2 * R, k0);
-        scores(k1, t0 + R, q, ksub, sub_lo, scale, sc, m);
-      }
+    scores(k0, 0, q, ksub, sub_lo, scale, sc, m);
+    for (int t0 = R; t0 < T; t0 += R) {
+      load_k(t0, k0);
+      scores(k0, t0, q, ksub, sub_lo, scale, sc, m);
     }
-    constexpr int RV = 2 * VB * C;
-    u32x4 v1[RING > 1 ? VU : 1];
-    if constexpr (RING > 1)
-      if (T > RV) load_v(RV, v1);  // in flight during the softmax
     m = wave_max(m);
     if (lane == 0) red_m[wave] = m;
     __syncthreads();  // also orders the sc writes before the reads below
@@ -292,24 +267,11 @@ struct HeadAttention {
     for (int u = 0; u < NU; ++u)
 #pragma unroll
       for (int e = 0; e < 8; ++e) acc[u][e] = 0.f;
-    if constexpr (RING == 1) {
-      values(v0, 0, vsub, sub_lo, sc, inv, acc);
-      for (int t0 = RV; t0 < T; t0 += RV) {
-        load_v(t0, v0);
-        values(v0, t0, vsub, sub_lo, sc, inv, acc);
-      }
-    } else {
-      for (int t0 = 0;; t0 += 2 * RV) {
-        values(v0, t0, vsub, sub_lo, sc, inv, acc);
-        if (t0 + RV >= T) break;
-        if (t0 + 2 * RV >= T) {
-          values(v1, t0 + RV, vsub, sub_lo, sc, inv, acc);
-          break;
-        }
-        load_v(t0 + 2 * RV, v0);
-        values(v1, t0 + RV, vsub, sub_lo, sc, inv, acc);
-        if (t0 + 3 * RV < T) load_v(t0 + 3 * RV, v1);
-      }
+    constexpr int RV = 2 * VB * C;
+    values(v0, 0, vsub, sub_lo, sc, inv, acc);
+    for (int t0 = RV; t0 < T; t0 += RV) {
+      load_v(t0, v0);
+      values(v0, t0, vsub, sub_lo, sc, inv, acc);
     }
     // the thread's classes, then the wave's lanes (lane bits LV ..)
 #pragma unroll
@@ -441,7 +403,7 @@ __global__ __launch_bounds__(kAttnThreads, 8) void attention_kernel(const uint16
                                                                  uint16_t* __restrict__ out, int max_len,
                                                                  float scale) {
   constexpr int D = 8 * LPR;
-  using Att = HeadAttention<LPR, 1, false, 1>;
+  using Att = HeadAttention<LPR, 1, false>;
   __shared__ float sc[AttnShape<LPR>::PLEN];
   __shared__ float part[Att::PART];
   __shared__ __align__(16) uint16_t qs[D];
@@ -502,7 +464,7 @@ __global__ __launch_bounds__(kAttnThreads) void rope_attention_kernel(const uint
   constexpr int D = 8 * LPR;
   constexpr int half = D / 2;
   constexpr int S = AttnShape<LPR>::SMAX;
-  using Att = HeadAttention<LPR, S, true, 2>;
+  using Att = HeadAttention<LPR, S, true>;
   __shared__ float sc[AttnShape<LPR>::PLEN];
   __shared__ float part[Att::PART];
   __shared__ __align__(16) uint16_t qs[D];
@@ -596,7 +558,7 @@ __global__ __launch_bounds__(kAttnThreads) void rope_attention_rows_kernel(const
                                                                            int max_len, float eps, float scale) {
   constexpr int D = 8 * LPR;
   constexpr int half = D / 2;
-  using Att = HeadAttention<LPR, 1, true, 2>;
+  using Att = HeadAttention<LPR, 1, true>;
   __shared__ float sc[AttnShape<LPR>::PLEN];
   __shared__ float part[Att::PART];
   __shared__ __align__(16) uint16_t qs[D];
