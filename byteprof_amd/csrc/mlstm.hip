@@ -372,7 +372,8 @@ __global__ __launch_bounds__(kMaxWaves * kWave) void mlstm_multistep_kernel(
 // no reduction. What bounds it is latency: with a position's gates, k and v loaded in its turn of the loop (and the
 // gates' exp and log in the chain) a position took 0.4 us. So lane l computes the activations of position l, only the
 // additions and maxima of m run in order, and the next eight positions' k and v are loaded during this eight's
-// arithmetic: 21 of 33 positions of 16 heads of 64 x 128 in bf16 11.2 -> 5.8 us.
+// arithmetic, where there are any: 21 of 33 positions of 16 heads of 64 x 128 in bf16 11.2 -> 5.6 us, one position 3.9 ->
+// 3.1 (a single workgroup pays 0.3 us for the wider first load: one head of 64 x 16 2.6 -> 2.9).
 // Reference semantics: byteprof/optim/mlstm_multistep.py:89-134 (lazy_commit_kernel), draft_fused.py:43-56.
 template <int IO, int BV, int DPT>
 __global__ __launch_bounds__(kMaxWaves * kWave) void mlstm_lazy_commit_kernel(
@@ -445,7 +446,7 @@ __global__ __launch_bounds__(kMaxWaves * kWave) void mlstm_lazy_commit_kernel(
       const float fa_l = round_io<IO>(__expf(fl + m_old - m_new));
       const float ia_l = round_io<IO>(__expf(iv - m_new));
       for (int g0 = 0; g0 < cnt; g0 += GP) {
-        load_group(next, c0 + g0 + GP);  // in flight during this group's arithmetic
+        if (c0 + g0 + GP < npos) load_group(next, c0 + g0 + GP);  // in flight during this group's arithmetic
         const float v_l = raw_value<IO>(cur.v);
         const int gcount = min(GP, cnt - g0);
 #pragma unroll

@@ -60,6 +60,35 @@ def test_lazy_commit_in_a_graph_with_a_dynamic_length(dtype, nh, dq, dv):
             assert err < tol, (length_v, err)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("nh,dq,dv,bv", [(3, 64, 32, 4), (2, 256, 48, 16), (1, 512, 16, 8)])
+def test_lazy_commit_of_many_positions_equals_the_steps(dtype, nh, dq, dv, bv):
+    """Rounds of several groups of loads (8 positions, 4 at bv 16) and of several chunks of gates (64): the state after
+    L + 1 of 9, 33, 65 and 130 positions equals, bit for bit, the one that as many single steps leave; one position
+    against the oracle."""
+    q, k, v, i, f, state = rand_inputs(130, nh, dq, dv, dtype, seed=5, f_mean=2.0)
+    states, prev = [], tuple(x.clone() for x in state)
+    h = torch.zeros(1, nh, dv, dtype=dtype, device="cuda")
+    for t in range(130):
+        new = tuple(torch.empty_like(x) for x in state)
+        DC.mlstm_step_into(prev, new, *(x[t:t + 1].contiguous() for x in (q, k, v, i, f)), h, 1e-6, bv=bv)
+        states.append(new)
+        prev = new
+    want = _oracle_state(state, k, v, i, f, 0, IO[dtype])
+    for got, ref in zip(states[0], want):
+        assert ON.normwise_error(got.cpu().numpy().reshape(ref.shape), ref) < (1e-5 if dtype == torch.float32 else 1e-2)
+    ns, ms = state[1][0].clone(), state[2].reshape(-1).clone()
+    for t in (9, 33, 65, 130):
+        kt, vt, it, ft = (x[:t].contiguous() for x in (k, v, i, f))
+        for length in sorted({0, 3, 6, 7, 8, 31, 32, 62, 63, 64, t - 2, t - 1}):
+            if length >= t:
+                continue
+            cur = tuple(x.clone() for x in state)
+            F.lazy_commit(cur, kt, vt, it, ft, torch.tensor(length, device="cuda"), ns, ms, bv=bv)
+            for got, ref in zip(cur, states[length]):
+                assert torch.equal(got.reshape(-1), ref.reshape(-1)), (t, length)
+
+
 def test_lazy_commit_with_no_accepted_position_keeps_the_start_state():
     q, k, v, i, f, state = rand_inputs(4, 4, 128, 64, torch.bfloat16, seed=1)
     cur = tuple(x.clone() for x in state)
