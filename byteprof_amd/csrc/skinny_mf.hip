@@ -103,15 +103,22 @@ int mf_nseg_wave(int64_t nseg, int waves, int split, int xstage, int wr) {
 
 // Whether a vector launch without a prologue takes the kernel of skinny_wide.h (the same sums, bit for bit). Measured
 // both ways on one MI355X (us, this kernel / the wide one):
-//   - past 10 rows always (16 rows: 2048 x 2048 bf16 5.4 / 5.3, 8192 x 2048 10.3 / 9.6; int8 100352 x 2048 57 / 43);
-//   - at 9 and 10 rows, not where the straight-line kernels keep more CUs at work (8-row workgroups: 2048 x 2048 at 9
-//     rows bf16 5.0 / 5.3, int8 4.5 / 5.1; 2048 x 8192 bf16 12.1 / 12.6, int8, 8 segments a wave, 9.2 / 8.8) or share
-//     staged rows between row groups in bf16 (16384 x 2048 15.9 / 16.5; int8 11.8 / 9.3);
-//   - up to 8 rows never (8 rows: 16000 x 1984 bf16 12.7 / 13.1, 1152 x 1152 3.6 / 4.4).
-bool mf_wide_takes(int wkind, int64_t M, int64_t N, int split, int nseg_wave, int wr) {
+//   - up to 8 rows never (8 rows: 16000 x 1984 bf16 12.7 / 13.1, 1152 x 1152 3.6 / 4.4), past 16 always, and where the
+//     waves' segments are not a straight-line count;
+//   - up to 2048 weight rows (8-row workgroups then keep every CU at work, 16 x 16 tiles half of them) not up to 16 rows
+//     (2048 x 2048 bf16 4.5 / 5.4 at 11 rows, 5.2 / 5.5 at 16; int8 4.4 / 5.2 and 4.7 / 5.3), but for int8 with 8 waves of
+//     more than 4 segments from 13 rows on (2048 x 8192 at 11 rows 8.7 / 9.0, at 16 10.5 / 10.0; with 4 waves 10.5 / 12.5);
+//   - past them from 11 rows on (3072 x 2048 bf16 6.1 / 5.8, 8192 x 2048 at 16 rows 10.3 / 9.6; int8 100352 x 2048 57 /
+//     43); at 9 and 10 rows not under 4096 weight rows (3072 x 1024 bf16 4.3 / 4.6) but for int8 with more than 4 segments
+//     a wave (3072 x 8192 13.0 / 10.4), nor where bf16 row groups share the staged rows (16384 x 2048 15.9 / 16.5; int8
+//     11.8 / 9.3).
+bool mf_wide_takes(int wkind, int64_t M, int64_t N, int waves, int split, int nseg_wave, int wr) {
   if (M <= 8) return false;
-  if (M > 10 || nseg_wave == 0) return true;
-  if (N * split < 4096) return wkind == kInt8 && nseg_wave > 4;
+  if (M > 16 || nseg_wave == 0) return true;
+  const bool long_int8 = wkind == kInt8 && nseg_wave > 4;
+  if (N * split <= 2048) return long_int8 && waves == 8 && M > 12;
+  if (M > 10) return true;
+  if (N * split < 4096) return long_int8;
   return !(wkind == kBf16 && wr > 1);
 }
 
@@ -232,7 +239,7 @@ int mf_launch(int wkind, const void* x, const void* w, const void* scale, int sc
   if (!menu(wr)) return BP_E_UNSUPPORTED;
   if (split > 1 && (ws == nullptr || ws_bytes < static_cast<size_t>(split) * M * N * sizeof(float)))
     return BP_E_WORKSPACE;
-  if (vec && pro.kind == 0 && mf_wide_takes(wkind, M, N, split, nseg_wave, wr))
+  if (vec && pro.kind == 0 && mf_wide_takes(wkind, M, N, waves, split, nseg_wave, wr))
     return mf_wide_launch(wkind, x, w, scale, scale_dt, y, M, N, K, waves, split, ws, st, mode);
   const MfFn fn = mf_pick(wkind, mf_blocks(M), rb, waves, vec, mode == 2 ? 1 : 0, xstage != 0, pro.kind != 0, nseg_wave,
                           wr);
@@ -349,7 +356,7 @@ int bp_skinny_mf_wide(int wkind, int64_t M, int64_t N, int64_t K, int waves, int
   if (K % seg != 0 || K >= bp::kMaxVecK) return 0;
   if (split > nseg) split = static_cast<int>(nseg);
   const int wr = bp::mf_row_groups(xstage);
-  if (!bp::mf_wide_takes(wkind, M, N, split, bp::mf_nseg_wave(nseg, waves, split, xstage, wr), wr)) return 0;
+  if (!bp::mf_wide_takes(wkind, M, N, waves, split, bp::mf_nseg_wave(nseg, waves, split, xstage, wr), wr)) return 0;
   const bp::MfWideTile t = bp::mf_wide_tile(wkind, M, N, split);
   return 256 * t.rp + t.mb;
 }

@@ -53,7 +53,7 @@ size_t bp_skinny_workspace_bytes(int64_t M, int64_t N, int split);
  *   BP_DT_BF16 / F16 / F32 on the fp32 sum), 1 <= M <= 64 per call (M = 0 or N = 0: no-op; K = 0: zeros).
  * One load instruction reads a 128-byte segment of 8 consecutive weight rows (one full line per row); the
  * activations are the MFMA's B operand (8 activation rows per 16 columns, the other 8 columns carry the other half of
- * the segment's K slots); past 8..10 rows a kernel with 16 x 16 blocks takes over (bp_skinny_mf_wide), which picks its
+ * the segment's K slots); from 9 to 17 rows on (by sizes) a kernel with 16 x 16 blocks takes over (bp_skinny_mf_wide), which picks its
  * own tile and ignores rb and xstage. Tile configuration: rb = 8-row weight blocks per workgroup (1, 2, 4; 4 up to
  * M = 16), waves = wavefronts sharing the workgroup's K segments (1, 2, 4, 8; segment s to wave s % waves), split = K ranges
  * in separate workgroups whose fp32 partials are added in split order by a second kernel (workspace as for

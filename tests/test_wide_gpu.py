@@ -66,18 +66,93 @@ def test_silu_rows_equal_the_one_row_kernel(kind, ffn):
         assert torch.equal(silu(x[:m].contiguous()).view(torch.int16), ones[:m].view(torch.int16)), m
 
 
-def test_the_rule_takes_every_tile_it_may_pick():
-    """Every tile of the rule is compiled for every wave count: a launch of each row count at sizes on both sides of its
-    lines returns success, and the rule never sends 8 rows or fewer to the wide kernel."""
-    L = _lib.lib()
-    for kind in (0, 1):
-        seg = 64 if kind == 0 else 128
-        for n in (1, 300, 2048, 4096, 6144, 16384, 100352):
-            for m in (1, 8, 9, 10, 11, 17, 33, 49, 64):
-                for waves in (1, 2, 4, 8):
-                    code = L.bp_skinny_mf_wide(kind, m, n, 32 * seg, waves, 1, 0)
-                    assert (code == 0) if m <= 8 else (code // 256 in (0, 1, 2, 4) and code % 256 <= 4)
-                    assert m <= 10 or code > 0
+def _rows(kind, x, args, waves, split, epi):
+    """bp_skinny_mf_rows of all rows of x in one call."""
+    m, k = x.shape
+    n = args[0].shape[0] // (1 + epi)
+    y = torch.full((m, n), 7.0, dtype=torch.bfloat16, device=DEV)
+    ws = torch.empty(max(1, split * m * n), dtype=torch.float32, device=DEV)
+    sc, sdt = (args[1].data_ptr(), _lib.TORCH_DT[args[1].dtype]) if kind == "int8" else (None, 0)
+    _lib.check(_lib.lib().bp_skinny_mf_rows(S._KIND_CODE[kind], x.data_ptr(), args[0].data_ptr(), sc, sdt, y.data_ptr(), m,
+                                            n, k, waves, split, epi, ws.data_ptr(), ws.numel() * 4,
+                                            _lib.stream_ptr(DEV)), "bp_skinny_mf_rows")
+    return y
+
+
+def _by_eight(kind, x, args, waves, split, epi):
+    """The same rows eight at a time: launches of the 8-row kernel."""
+    return torch.cat([_rows(kind, x[r:r + 8].contiguous(), args, waves, split, epi) for r in range(0, x.shape[0], 8)])
+
+
+@pytest.mark.parametrize("kind", ["bf16", "int8"])
+@pytest.mark.parametrize("waves", [1, 2, 4, 8])
+def test_every_tile_of_the_rule_runs_and_equals_the_8_row_kernel(kind, waves):
+    """Every (rp, mb) tile that the rule picks for 17..64 rows of any number of weight rows is compiled for every wave
+    count and both epilogues: launched once at the smallest size that has it, each row equal bit for bit to the 8-row
+    kernel's, and the plain product to the oracle. The rule never sends 8 rows or fewer to the wide kernel."""
+    L, code, seg = _lib.lib(), S._KIND_CODE[kind], S.k_segment(kind)
+    k = 2 * waves * seg  # two segments a wave: no straight-line kernel
+    tiles = {}
+    for n in (2, 30, 300, 2048, 4096, 6144, 8192, 12000, 16384, 20000, 33000):
+        assert all(L.bp_skinny_mf_wide(code, m, n, k, waves, 1, 0) == 0 for m in range(1, 9))
+        for m in range(9, 65):
+            t = L.bp_skinny_mf_wide(code, m, n, k, waves, 1, 0)
+            assert t > 0 and t // 256 in (1, 2, 4) and 1 <= t % 256 <= 4, (n, m, t)
+            if t not in tiles or n * m < tiles[t][0] * tiles[t][1]:
+                tiles[t] = (n, m)
+    assert {t // 256 for t in tiles} == {1, 2, 4}, tiles
+    for t, (n, m) in tiles.items():
+        _, args = make_weights(kind, n, k, seed=n + m)
+        x = randn_x(m, k, seed=m)
+        for epi in (0, 1):
+            if epi == 1 and m <= 16:  # the SiLU launches of up to 16 rows: test_silu_rows_equal_the_one_row_kernel
+                continue
+            got, want = _rows(kind, x, args, waves, 1, epi), _by_eight(kind, x, args, waves, 1, epi)
+            assert torch.equal(got.view(torch.int16), want.view(torch.int16)), (t, n, m, epi)
+        if n <= 2048:
+            check_against_oracle(_rows(kind, x, args, waves, 1, 0), x, oracle_weights(kind, args))
+
+
+@pytest.mark.parametrize("kind", ["bf16", "int8"])
+@pytest.mark.parametrize("n,segs,waves,split,epi", [(70, 5, 4, 1, 0), (70, 5, 4, 1, 1), (1030, 9, 2, 2, 0),
+                                                    (6150, 4, 4, 1, 1), (6150, 8, 8, 2, 0)])
+def test_mf_rows_past_64_rows(kind, n, segs, waves, split, epi):
+    """bp_skinny_mf_rows, one launch for a prompt's rows: 5 to 16 activation blocks, several activation tiles per weight
+    tile, a last one of one row, the split reduce over all rows; each row equal bit for bit to the 8-row kernel's."""
+    k = segs * S.k_segment(kind)
+    _, args = make_weights(kind, n, k, seed=n)
+    x = randn_x(256, k, seed=segs)
+    want = _by_eight(kind, x, args, waves, split, epi)
+    for m in (65, 97, 127, 160, 255, 256):
+        got = _rows(kind, x[:m].contiguous(), args, waves, split, epi)
+        assert torch.equal(got.view(torch.int16), want[:m].view(torch.int16)), m
+
+
+@pytest.mark.parametrize("n,groups,tile,waves,split,epi", [(70, 5, 16, 4, 1, 0), (300, 9, 32, 8, 2, 0), (300, 3, 32, 2, 1, 1),
+                                                           (4100, 4, 64, 1, 1, 0), (22, 3, 16, 4, 1, 0)])
+def test_int4_rows_past_64_rows(n, groups, tile, waves, split, epi):
+    """bp_skinny_int4_rows past 64 rows, the VALU kernel's shapes (n % 4 != 0: 16 rows a launch inside) among them."""
+    k = groups * S.GROUP
+    w = (torch.randn(n * (1 + epi), k, generator=torch.Generator(device=DEV).manual_seed(n), device=DEV) * 0.02).to(
+        torch.bfloat16)
+    packed, scale, zero = S.quantize_int4(w, tile)
+    x = randn_x(256, k, seed=n)
+    ws = torch.empty(split * 256 * n, dtype=torch.float32, device=DEV)
+
+    def rows(xm):
+        y = torch.full((xm.shape[0], n), 7.0, dtype=torch.bfloat16, device=DEV)
+        _lib.check(_lib.lib().bp_skinny_int4_rows(xm.data_ptr(), packed.data_ptr(), scale.data_ptr(),
+                                                  _lib.TORCH_DT[scale.dtype], zero.data_ptr(), y.data_ptr(), xm.shape[0], n,
+                                                  k, tile, waves, split, epi, ws.data_ptr(), ws.numel() * 4,
+                                                  _lib.stream_ptr(DEV)), "bp_skinny_int4_rows")
+        return y
+
+    ones = torch.cat([rows(x[r:r + 1].contiguous()) for r in range(256)])
+    for m in (65, 97, 127, 160, 255, 256):
+        got = rows(x[:m].contiguous())
+        assert torch.equal(got.view(torch.int16), ones[:m].view(torch.int16)), m
+    if epi == 0:
+        check_against_oracle(ones, x, S.dequantize("int4", packed, scale, zero).cpu().numpy())
 
 
 @pytest.mark.parametrize("tile_rows", [16, 32, 64])
