@@ -13,8 +13,10 @@ loop), and at one row with a norm prologue (split 1). It keeps the fastest one-r
 split > 1 must win by more than 3%; when that order has no split, the split-1 order within 5% of it whose plain and
 prologue launches are fastest together (the decode step runs the prologue form); then, among the orders within 2%
 of that, the fastest at 16 rows. Then, at that K order, it picks the weight blocks per workgroup and
-the flags for each bucket (1; 8: four and eight rows together; 16: nine and sixteen rows, the row groups over one
-staged copy among its plans; 32, 64; `--plans-only 16` retunes just those buckets in an existing table). Last, for
+the flags for each bucket whose launches use them (1; 8: four and eight rows together; 16: nine and sixteen, the row groups over
+one staged copy among its plans). The wide kernel picks its own tile and ignores both: the buckets of its launches (all
+past 16 rows) are timed once and hold rb 1, xs 0 (`--plans-only 16` retunes just those buckets in an existing table; for int4 it times the
+entry's plan again). Last, for
 launches with a norm prologue (bp_skinny_mf_pro: the decode loops' q|k|v, gate|up and LM head launches), the weight
 blocks per workgroup at the same K order, for buckets 1 and 8 (rb_pro; `--pro-only` retunes just those).
 
@@ -115,9 +117,20 @@ def _plans(kind: str, m: int, k: int, waves: int, split: int):
                 yield rb, xs
 
 
+def _wide(kind, m, n, k, waves, split) -> bool:
+    """Whether a launch of m rows runs the wide kernel under every plan (all past 16 rows, many from 9 on)."""
+    from . import _lib
+
+    plans = (0, S.XS_STAGE | S.XS_ROWS2, S.XS_STAGE | S.XS_ROWS4)
+    return all(_lib.lib().bp_skinny_mf_wide(S._KIND_CODE[kind], m, n, k, waves, split, xs) for xs in plans)
+
+
 def _best_plan(kind, ring, x, y, waves, split, rows_list) -> tuple[float, int, int]:
-    """(summed us over the row counts, rb, staging) of the best plan at this K order."""
+    """(summed us over the row counts, rb, staging) of the best plan at this K order; where every row count runs the wide
+    kernel, one plan stands for all."""
     best = None
+    if all(_wide(kind, m, y.shape[1], x.shape[1], waves, split) for m in rows_list):
+        return sum(_time_calls(_launcher(kind, ring, x[:m].contiguous(), y[:m], 1, waves, split, 0)) for m in rows_list), 1, 0
     for rb, xs in _plans(kind, max(rows_list), x.shape[1], waves, split):
         t = sum(_time_calls(_launcher(kind, ring, x[:m].contiguous(), y[:m], rb, waves, split, xs))
                 for m in rows_list)
@@ -126,10 +139,16 @@ def _best_plan(kind, ring, x, y, waves, split, rows_list) -> tuple[float, int, i
     return best
 
 
+def _in_turn(a, b, rounds: int = 5) -> tuple[float, float]:
+    """us of two timings (functions) taken in turn: the medians over the rounds, which the card's drift then shares."""
+    ta, tb = zip(*((a(), b()) for _ in range(rounds)))
+    return statistics.median(ta), statistics.median(tb)
+
+
 PRO_BUCKETS = {1: (1,), 8: (2, 4)}  # the row buckets (and row counts timed) where the decode loops run norm prologues
 
 
-def tune_pro(kind: str, n: int, k: int, entry: dict, device, log=print) -> dict:
+def tune_pro(kind: str, n: int, k: int, entry: dict, device, log=print, held: dict | None = None) -> dict:
     """rb_pro: the weight blocks per workgroup of launches with a norm prologue (bp_skinny_mf_pro, BP_PRO_NORM with
     a residual, as the decode step's q|k|v, gate|up and LM head launches run) at the table's K order, per row bucket
     where the rows stage in LDS; {} where the order splits K (no prologue there)."""
@@ -147,10 +166,7 @@ def tune_pro(kind: str, n: int, k: int, entry: dict, device, log=print) -> dict:
     for bucket, rows in PRO_BUCKETS.items():
         if S._stage_bytes(kind, max(rows), k, 1) < 0:  # the rows must stage in LDS
             continue
-        best = None
-        for rb in RBS:
-            if not S._supported(kind, max(rows), rb, waves, True):
-                continue
+        def total(rb):
             t = 0.0
             for m in rows:
                 calls = [lambda a=a, m=m: S.prologue_mm(x[:m], a[0], a[1] if kind == "int8" else None, y[:m],
@@ -158,10 +174,18 @@ def tune_pro(kind: str, n: int, k: int, entry: dict, device, log=print) -> dict:
                                                         eps=1e-6, cfg=(8 * rb, waves, 1))
                          for a in ring]
                 t += _time_calls(calls)
-            if best is None or t < best[0]:
-                best = (t, rb)
-        if best is not None:
-            out[str(bucket)] = best[1]
+            return t
+
+        rbs = [rb for rb in RBS if S._supported(kind, max(rows), rb, waves, True)]
+        if not rbs:
+            continue
+        best = min(rbs, key=total)
+        was = (held or {}).get(str(bucket))
+        if was in rbs and was != best:
+            t_new, t_held = _in_turn(lambda: total(best), lambda: total(was))
+            if t_new > 0.985 * t_held:  # the table's stays unless the new one is 1.5% faster
+                best = was
+        out[str(bucket)] = best
     log(f"  {kind} {n}x{k}: rb_pro={out}")
     del ring
     torch.cuda.empty_cache()
@@ -206,6 +230,16 @@ def retune_plans(kind: str, n: int, k: int, entry: dict, buckets, device, log=pr
         if bucket not in buckets:
             continue
         _, rb, xs = _best_plan(kind, ring, x, y, waves, split, rows)
+        held = (entry.get("rb", {}).get(str(bucket)), entry.get("xs", {}).get(str(bucket), 0))
+        wide = all(_wide(kind, m, n, k, waves, split) for m in rows)
+        if not wide and held[0] is not None and held != (rb, xs) and held in set(_plans(kind, max(rows), k, waves, split)):
+            def total(plan):
+                return sum(_time_calls(_launcher(kind, ring, x[:m].contiguous(), y[:m], plan[0], waves, split, plan[1]))
+                           for m in rows)
+
+            t_new, t_held = _in_turn(lambda: total((rb, xs)), lambda: total(held))
+            if t_new > 0.985 * t_held:  # the table's plan stays unless the new one is 1.5% faster
+                rb, xs = held
         out["rb"][str(bucket)], out["xs"][str(bucket)] = rb, xs
         for m in rows:
             out["us"][str(m)] = round(_time_calls(_launcher(kind, ring, x[:m].contiguous(), y[:m], rb, waves, split,
@@ -266,6 +300,32 @@ def tune_shape(kind: str, n: int, k: int, device, log=print) -> dict:
     return {"waves": waves, "split": split, "rb": rb, "xs": xs, "us": us, **({"rb_pro": rb_pro} if rb_pro else {})}
 
 
+INT4_US_ROWS = (1, 2, 4, 8, 16)
+
+
+def _int4_ring(n: int, k: int, tile_rows: int, device) -> list[tuple]:
+    count = max(2, min(64, RING_BYTES // (n * k // 2)))
+    g = torch.Generator(device=device).manual_seed(n * 17 + k)
+    ring = []
+    for _ in range(count):
+        w = (torch.randn(n, k, generator=g, device=device) * 0.02).to(torch.bfloat16)
+        ring.append(S.quantize_int4(w, tile_rows))
+        del w
+    return ring
+
+
+def time_int4(n: int, k: int, tile_rows: int, plan, device, ring=None) -> tuple[dict, list]:
+    """us per row count of an int4 weight in tiles of tile_rows at plan (waves, split), and the ring of weights."""
+    ring = ring or _int4_ring(n, k, tile_rows, device)
+    x = torch.randn(max(INT4_US_ROWS), k, device=device).to(torch.bfloat16)
+    y = torch.empty(max(INT4_US_ROWS), n, dtype=torch.bfloat16, device=device)
+    us = {}
+    for m in INT4_US_ROWS:
+        xb, yb = x[:m].contiguous(), y[:m]
+        us[str(m)] = round(_time_calls([lambda a=a: S.skinny_mm(xb, *a, out=yb, cfg=plan) for a in ring]), 3)
+    return us, ring
+
+
 def tune_int4(n: int, k: int, device, log=print, tiles=S.INT4_TILES) -> dict | None:
     """int4: per tile rows (16, 32, 64: a packing choice), (waves, split) by the M = 1 time (split > 1 kept only if
     it wins by more than 3%); the tile rows of the fastest plan are the entry's, with the time of every row bucket
@@ -274,18 +334,11 @@ def tune_int4(n: int, k: int, device, log=print, tiles=S.INT4_TILES) -> dict | N
         return None
     groups = k // S.GROUP
     per = n * k // 2
-    count = max(2, min(64, RING_BYTES // per))
-    x16 = torch.randn(16, k, device=device).to(torch.bfloat16)
-    y = torch.empty(16, n, dtype=torch.bfloat16, device=device)
-    x1, y1 = x16[:1].contiguous(), y[:1]
+    x1 = torch.randn(1, k, device=device).to(torch.bfloat16)
+    y1 = torch.empty(1, n, dtype=torch.bfloat16, device=device)
     plans, best_tile, us = {}, None, {}
     for tr in tiles:
-        g = torch.Generator(device=device).manual_seed(n * 17 + k)
-        ring = []
-        for _ in range(count):
-            w = (torch.randn(n, k, generator=g, device=device) * 0.02).to(torch.bfloat16)
-            ring.append(S.quantize_int4(w, tr))
-            del w
+        ring = _int4_ring(n, k, tr, device)
         results = {}
         for w in INT4_WAVES:
             if w > groups:
@@ -303,10 +356,7 @@ def tune_int4(n: int, k: int, device, log=print, tiles=S.INT4_TILES) -> dict | N
         log(f"  int4 {n}x{k} tile {tr}: waves={best[0]} split={best[1]}: {results[best]:.3f} us at M=1")
         if best_tile is None or results[best] < plans[str(best_tile)]["us1"]:
             best_tile = tr
-            us = {}
-            for bm in (1, 2, 4, 8, 16):
-                xb, yb = x16[:bm].contiguous(), y[:bm]
-                us[str(bm)] = round(_time_calls([lambda a=a: S.skinny_mm(xb, *a, out=yb, cfg=best) for a in ring]), 3)
+            us, _ = time_int4(n, k, tr, best, device, ring)
         del ring
         torch.cuda.empty_cache()
     top = plans[str(best_tile)]
@@ -334,7 +384,8 @@ def main(argv=None) -> int:
                        "(bf16, int8): waves and split of the matrix-core kernel (they fix the K order for every row "
                        "count), rb = 8-row weight blocks per workgroup and xs = xstage flags (1: activations "
                        "staged in LDS, 2: the general segment loop instead of the straight-line kernel of the "
-                       "segment count), per row bucket (1, 8, 16, 32, 64), rb_pro = rb of launches with a norm "
+                       "segment count), per row bucket (1, 8, 16, 32, 64; the wide kernel, past 16 rows always, ignores both: "
+                       "1 and 0 there), rb_pro = rb of launches with a norm "
                        "prologue (buckets 1 and 8), us = measured time per call by row count (ring of distinct "
                        "weights, HIP graph); int4|N|K: tile_rows = the rows per tile to pack the weight "
                        "with, waves and split of the int4 kernel at those tile rows, us per row count, and tiles = the "
@@ -345,7 +396,13 @@ def main(argv=None) -> int:
         for kind in a.kinds.split(","):
             for n, k in shapes:
                 key = f"{kind}|{n}|{k}"
-                if kind == "int4" or key not in table:
+                if key not in table:
+                    continue
+                if kind == "int4":
+                    e = table[key]
+                    e["us"], _ = time_int4(n, k, e["tile_rows"], (e["waves"], e["split"]), device)
+                    print(f"[tune] {key} us {e['us']}", flush=True)
+                    out.write_text(json.dumps(table, indent=1, sort_keys=True) + "\n")
                     continue
                 print(f"[tune] {key} plans of buckets {sorted(buckets)}", flush=True)
                 table[key] = retune_plans(kind, n, k, table[key], buckets, device, log=log)
@@ -359,7 +416,7 @@ def main(argv=None) -> int:
                 if kind == "int4" or key not in table:
                     continue
                 print(f"[tune] {key} rb_pro", flush=True)
-                rb_pro = tune_pro(kind, n, k, table[key], device, log=log)
+                rb_pro = tune_pro(kind, n, k, table[key], device, log=log, held=table[key].get("rb_pro", {}))
                 if rb_pro:
                     table[key]["rb_pro"] = rb_pro
                 else:
