@@ -333,17 +333,22 @@ def _deq4(args) -> np.ndarray:
 # hidden sizes that are not whole segments (64 bf16 or 128 int8 elements), and an int4 vocabulary off the groups of four
 RAGGED = {"h224": OG.OlmoConfig(hidden=224, ffn=512, layers=2, heads=7, vocab=512, max_len=96),
           "h448": OG.OlmoConfig(hidden=448, ffn=896, layers=2, heads=7, vocab=512, max_len=96),
-          "v1001": OG.OlmoConfig(hidden=128, ffn=256, layers=2, heads=2, vocab=1001, max_len=96)}
+          "v1001": OG.OlmoConfig(hidden=128, ffn=256, layers=2, heads=2, vocab=1001, max_len=96),
+          # ragged and long enough that the default plans split K in every linear
+          "h2080": OG.OlmoConfig(hidden=2080, ffn=2100, layers=1, heads=65, vocab=512, max_len=96)}
 
 
 @pytest.mark.parametrize("kind,shape", [("bf16", "h224"), ("bf16", "h448"), ("int8", "h224"), ("int8", "h448"),
-                                        ("int4", "v1001")])
+                                        ("int4", "v1001"), ("bf16", "h2080")])
 def test_ragged_decoders_match_the_oracle(kind, shape):
     """Decoders whose linears take the element loads (no epilogue, no prologue) or the int4 VALU kernel: the steps against
     the oracle, the prompt passes against the steps, and a verify pass against the steps."""
     cfg = RAGGED[shape]
     dec, W, oc = _small_decoder(kind, cfg=cfg)
     assert dec.fuse_norms == all(dec._whole_rows(n, cfg.hidden, 1) for n in (3 * cfg.hidden, 2 * cfg.ffn, cfg.vocab))
+    if shape == "h2080":
+        assert all(dec._plan(n, k, 1)[2] > 1 for n, k in ((3 * 2080, 2080), (2080, 2080), (4200, 2080), (2080, 2100),
+                                                          (512, 2080))) and dec._down_splitk(3) is not None
     prompt = [3, 17, 99, 250, 7] * 8
     toks, logits = OO.greedy(W, oc, prompt, 4)
     dec.pos.zero_()

@@ -52,6 +52,33 @@ def test_row_groups_equal_the_plain_kernel_bit_for_bit(kind, n, k):
     assert ran > 0  # the menu holds row-group kernels for these shapes
 
 
+@pytest.mark.parametrize("kind", ["bf16", "int8"])
+@pytest.mark.parametrize("n,k", [(2048, 2048), (1001, 1024), (520, 4096)])
+def test_8_row_kernel_at_9_to_16_rows_equals_the_rows_one_by_one(kind, n, k):
+    """Up to 2048 weight rows the 8-row kernel runs 9..16 rows: every compiled (rb, waves, staging, row groups) of it that a
+    launch takes (the wide kernel takes the others and ignores all but the waves), against one-row launches."""
+    _, args = make_weights(kind, n, k, seed=n + k)
+    x = randn_x(16, k, seed=k)
+    ran = set()
+    for waves in (2, 4, 8):
+        one = torch.cat([_launch(kind, args, x[i:i + 1], n, 1, waves, 0) for i in range(16)])
+        for m in (9, 12, 16):
+            for xs in (0, S.XS_STAGE, S.XS_STAGE | S.XS_ROWS2, S.XS_STAGE | S.XS_ROWS4):
+                for rb in (1, 2, 4):
+                    if not S._supported(kind, m, rb, waves, xs) or (xs and S._stage_bytes(kind, m, k, 1, xs) < 0):
+                        continue
+                    if _lib.lib().bp_skinny_mf_wide(S._KIND_CODE[kind], m, n, k, waves, 1, xs):
+                        continue
+                    y = _launch(kind, args, x[:m], n, rb, waves, xs)
+                    assert torch.equal(y, one[:m]), (m, waves, rb, xs)
+                    ran.add((rb, waves, xs))
+    check_against_oracle(one, x, oracle_weights(kind, args))
+    print(f"\n[rows] {kind} n={n} k={k}: {sorted(ran)}", flush=True)
+    assert len(ran) >= 5 and any(xs == 0 for _, _, xs in ran)
+    if k <= 2048 and kind == "bf16":
+        assert any(xs & S.XS_ROWS for _, _, xs in ran)
+
+
 def test_row_group_flags_are_ignored_outside_their_plans(monkeypatch):
     """At 8 rows or fewer, without staging, or past the 64 KiB staging limit, a plan with row-group flags resolves
     to a plan without them (skinny_mm never launches an uncompiled row-group kernel)."""

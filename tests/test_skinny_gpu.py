@@ -268,7 +268,8 @@ FIXED_PLANS = [(2048, 2048, 8, 4, 1), (6144, 2048, 8, 2, 1), (2050, 2048, 16, 8,
 def test_straight_line_kernel_equals_the_general_loop(kind, n, k, rows, waves, split):
     """A launch whose waves all have 4, 8 or 16 segments runs the straight-line kernel of that count; with
     BP_XS_GENERAL the same plan runs the general segment loop. Same segments in the same order: equal bit for bit,
-    with and without the LDS-staged activations, at 1..33 rows; and within the oracle's tolerance."""
+    with and without the LDS-staged activations; and within the oracle's tolerance. (From 9 rows on the general loop's plan
+    runs the wide kernel, which the straight-line kernel has to equal up to 16 rows; at 33 rows both are the wide kernel.)"""
     from byteprof_amd import _lib
 
     L = _lib.lib()
