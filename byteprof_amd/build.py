@@ -41,7 +41,8 @@ def common_flags() -> list[str]:
 
 
 SOURCES = ("skinny.hip", "skinny_mf.hip", "skinny_mf_n4.hip", "skinny_mf_n8.hip", "skinny_mf_n16.hip",
-           "skinny_wide.hip",           "skinny_chain.hip", "skinny_int4.hip", "skinny_int4_wide.hip", "mlstm.hip", "draft.hip", "decode.hip")
+           "skinny_wide.hip", "skinny_chain.hip", "skinny_int4.hip", "skinny_int4_wide.hip", "mlstm.hip", "draft.hip",
+           "decode.hip")
 
 
 def units() -> list[tuple[Path, list[str], Path]]:

@@ -80,8 +80,9 @@ constexpr int kAttnWaves = kAttnThreads / kWave;
 // are packed (v_dot2_f32_bf16, two of them an operation), a round's reductions share their steps, and S workgroups share
 // a head: each reads the head's whole K rows for the scores (they run on one XCD and meet in its L2), and only its own
 // columns of V. Launches of many rows have workgroups enough (S = 1). The order of every sum is the same for every S:
-//   - scores: LPR lanes per cache row (16 bytes each, whole lines), four row batches per round; a lane's 8 products by v_dot2_f32_bf16 in order, then a butterfly over the row's lanes (distances LPR/2
-//     .. 1) for the round's rows at once. s_t = bf16(bf16(q . k_t) * scale), p = bf16(softmax_fp32(s));
+//   - scores: LPR lanes per cache row (16 bytes each, whole lines), four row batches per round; a lane's 8 products by
+//     v_dot2_f32_bf16 in order, then a butterfly over the row's lanes (distances LPR/2 .. 1) for the round's rows at
+//     once. s_t = bf16(bf16(q . k_t) * scale), p = bf16(softmax_fp32(s));
 //   - values: position t belongs to class t % C (C = 512 SMAX / LPR). A thread adds its class's positions in order, two
 //     at a time (t and t + C: v_dot2_f32_bf16 on the pair); the classes are added as a tree over the bits of the class:
 //     the highest first (with S = 1 the two classes a thread holds, else a lane bit), then the lowest on, lanes by
@@ -99,7 +100,8 @@ struct AttnShape {
   static constexpr int PLEN = kAttnMaxLen + 2 * C;  // scores, then zeros up to whole pairs of classes
 };
 
-// Butterfly over lane distances DIST .. 1 of N values per lane at once (reduce_stage); first: the index of v[0] among the N.
+// Butterfly over lane distances DIST .. 1 of N values per lane at once (reduce_stage); first: the index of v[0] among the
+// N.
 template <int DIST, int N>
 __device__ __forceinline__ void reduce_rows(float* v, int lane, int& first) {
   if constexpr (DIST >= 1) {
@@ -218,7 +220,8 @@ struct HeadAttention {
         if (t + C >= sub_lo && t + C < T) b = *reinterpret_cast<const u32x4*>(vsub + (t + C - sub_lo) * D + vcol);
       }
       if (t < T) {
-        const uint32_t p = float_to_bf16_bits(sc[t] * inv) | (static_cast<uint32_t>(float_to_bf16_bits(sc[t + C] * inv)) << 16);
+        const uint32_t p = float_to_bf16_bits(sc[t] * inv) |
+                           (static_cast<uint32_t>(float_to_bf16_bits(sc[t + C] * inv)) << 16);
         float (&ac)[8] = acc[(u / 2) % NU];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
@@ -446,11 +449,11 @@ __device__ __forceinline__ void read_rows(const uint16_t* K, const uint16_t* V, 
   }
 }
 
-// qk_rope_cache and attention in one launch, SMAX workgroups per head (HeadAttention): every workgroup computes the q / k norms over the whole projections
-// (the same sums in every workgroup, in qk_rope_cache_kernel's order: the results are equal bit for bit to the two
-// launches), rotates its own head, the first of a head writes its k and v at pos to the cache, and each attends over positions
-// 0 .. pos with that row taken from LDS. Every load that does not depend on the norms (the projections, the RoPE
-// operands, the first batch of cache rows) is issued before the first reduction.
+// qk_rope_cache and attention in one launch, SMAX workgroups per head (HeadAttention): every workgroup computes the q / k
+// norms over the whole projections (the same sums in every workgroup, in qk_rope_cache_kernel's order: the results are
+// equal bit for bit to the two launches), rotates its own head, the first of a head writes its k and v at pos to the
+// cache, and each attends over positions 0 .. pos with that row taken from LDS. Every load that does not depend on the
+// norms (the projections, the RoPE operands, the first batch of cache rows) is issued before the first reduction.
 template <int LPR>
 __global__ __launch_bounds__(kAttnThreads) void rope_attention_kernel(const uint16_t* __restrict__ qkv,
                                                                       const uint16_t* __restrict__ qw,

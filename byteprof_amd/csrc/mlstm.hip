@@ -146,8 +146,9 @@ struct MlstmBlock {
   }
 };
 
-// G positions per reduction group: 64 / BV, or 1 for a launch of one position (the addition trees do not depend on how many
-// values share a reduction, so the same bits: a step of 4 heads of 256 x 256 in float32 5.4 us with groups of 16, 3.4 with one).
+// G positions per reduction group: 64 / BV, or 1 for a launch of one position (the addition trees do not depend on how
+// many values share a reduction, so the same bits: a step of 4 heads of 256 x 256 in float32 5.4 us with groups of 16,
+// 3.4 with one).
 template <int IO, int BV, int DPT, int G>
 __global__ __launch_bounds__(kMaxWaves * kWave) void mlstm_multistep_kernel(
     const float* __restrict__ c, const float* __restrict__ n, const float* __restrict__ m,

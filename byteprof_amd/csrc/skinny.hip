@@ -104,8 +104,8 @@ int skinny_int4_launch(const void* x, const void* packed, const void* scale, int
   if (reinterpret_cast<uintptr_t>(x) % 16 != 0 || reinterpret_cast<uintptr_t>(packed) % 16 != 0 ||
       reinterpret_cast<uintptr_t>(zero) % 2 != 0)
     return BP_E_UNSUPPORTED;
-  // the matrix-core kernel where a lane's four rows can read their scale and zero as one vector each, and the
-  // activations of up to 16 rows fit one buffer resource (K < 2^24); the choice does not depend on M
+  // the matrix-core kernels where a lane's four rows can read their scale and zero as one vector each, and a workgroup's
+  // activations (up to 32 rows) fit one buffer resource (K < 2^24); the choice does not depend on M
   const int64_t sc_align = scale_dt == BP_DT_F32 ? 16 : 8;
   const bool mf = N % 4 == 0 && reinterpret_cast<uintptr_t>(zero) % 8 == 0 &&
                   reinterpret_cast<uintptr_t>(scale) % sc_align == 0 && K < (int64_t{1} << 24);
@@ -116,8 +116,9 @@ int skinny_int4_launch(const void* x, const void* packed, const void* scale, int
   if (nb == 0 && M > 16) {  // the VALU kernel: 16 rows a launch
     for (int64_t r = 0; r < M; r += 16) {
       const int rc = skinny_int4_launch(static_cast<const uint16_t*>(x) + r * K, packed, scale, scale_dt, zero,
-                                        static_cast<uint16_t*>(y) + r * (epi != 0 ? N / 2 : N), std::min<int64_t>(16, M - r), N, K, tile_rows,
-                                        waves, split, ws, ws_bytes, stream, epi);
+                                        static_cast<uint16_t*>(y) + r * (epi != 0 ? N / 2 : N),
+                                        std::min<int64_t>(16, M - r), N, K, tile_rows, waves, split, ws, ws_bytes,
+                                        stream, epi);
       if (rc != BP_OK) return rc;
     }
     return BP_OK;

@@ -5,8 +5,8 @@
 
 namespace bp {
 
-// The int4 matrix-core kernel of 1..64 activation rows (skinny_int4_wide.hip): activation blocks of 16 per workgroup (nb:
-// 1, 2), tile rows, waves, scale dtype, epilogue (0: the product, 1: the gate|up SiLU product); or null.
+// The int4 matrix-core kernel of any number of activation rows (skinny_int4_wide.hip): activation blocks of 16 per
+// workgroup (nb: 1, 2), tile rows, waves, scale dtype, epilogue (0: the product, 1: the gate|up SiLU product); or null.
 using Int4WideFn = void (*)(const uint16_t*, const uint8_t*, const void*, const uint16_t*, uint16_t*, float*, int, int64_t,
                             int64_t, int);
 Int4WideFn int4_wide_pick(int nb, int tile_rows, int waves, int scale_dt, int epi);

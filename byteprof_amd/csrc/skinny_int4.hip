@@ -182,8 +182,8 @@ struct I4Slot {
 };
 
 // PRO (up to 8 activation rows, split 1): the rows staged in LDS with gamma, the residual rows and gamma2 (dynamic
-// shared memory, (2 M + 2) K bf16), transformed by mf_prologue (the norm kernel's arithmetic: the product equals a norm launch
-// followed by the plain kernel, bit for bit) while the first groups' weights are in flight; the B operands are then
+// shared memory, (2 M + 2) K bf16), transformed by mf_prologue (the norm kernel's arithmetic: the product equals a norm
+// launch followed by the plain kernel, bit for bit) while the first groups' weights are in flight; the B operands are then
 // read from LDS.
 template <int RB, int WAVES, int DEPTH, int SDT, int EPI = 0, bool PRO = false>
 __global__ __launch_bounds__(WAVES * kWave) void skinny_int4_mf_kernel(const uint16_t* __restrict__ x,

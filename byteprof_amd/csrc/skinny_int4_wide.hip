@@ -1,13 +1,13 @@
-// The int4 matrix-core kernel for up to 64 activation rows in one launch: skinny_int4.hip's groups, waves and sums (an
-// output is the same bits), with NB blocks of 16 activation rows as the MFMA's B columns, so a verify pass or a prompt of
-// more than 16 rows streams the codes and decodes them once (or once per 32 rows).
+// The int4 matrix-core kernel for any number of activation rows in one launch: skinny_int4.hip's groups, waves and sums
+// (an output is the same bits), with NB blocks of 16 activation rows as the MFMA's B columns, so a verify pass or a
+// prompt of more than 16 rows streams the codes and decodes them once (or once per 32 rows).
 //
 // What bounds it is the activations: a group is 1 KiB of codes per 16 weight rows, and 4 KiB of activations per 16
 // activation rows. They are loaded as whole 256-byte rows in lane order and turned into operands through the wave's own
 // LDS patch (16 rows x 128 K, pieces swizzled by the row, no barrier): loaded in operand order, with neighbouring lanes
-// in different rows, the address unit takes four times as long. us on one MI355X, before
-// (launches of 16 rows by skinny_int4.hip) -> now: 64 rows of 2048 x 2048 25.3 -> 5.7, 8192 x 2048 31.5 -> 10.9, 2048 x 8192
-// 50.1 -> 12.5, 100352 x 2048 120 -> 59; 16 rows 6.5 -> 4.2, 8.1 -> 5.3, 12.6 -> 8.9, 33.0 -> 26.3.
+// in different rows, the address unit takes four times as long. us on one MI355X, before (launches of 16 rows by
+// skinny_int4.hip) -> now: 64 rows of 2048 x 2048 25.3 -> 5.7, 8192 x 2048 31.5 -> 10.9, 2048 x 8192 50.1 -> 12.5, 100352 x
+// 2048 120 -> 59; 16 rows 6.5 -> 4.2, 8.1 -> 5.3, 12.6 -> 8.9, 33.0 -> 26.3.
 //
 // Reference semantics: byteprof/optim/skinny.py:46-63 (MODE 3 kernel), through skinny_mm (skinny.py:136-166).
 
@@ -57,7 +57,9 @@ __global__ __launch_bounds__(WAVES* kWave, 2) void skinny_int4_wide_kernel(
   const int64_t first = g_lo + wave;
   const int cnt = first < g_hi ? static_cast<int>((g_hi - first + WAVES - 1) / WAVES) : 0;
   const uint8_t* tile = w + tb * G * R * 64 + i * 64 + kb * 16;
-  // K < 2^24 and M <= 64: 2 M K < 2^31; a row past M has an offset past the resource (zeros, no memory request)
+  // K < 2^24 and M <= 16 NB <= 32 (the workgroup's rows): 2 M K < 2^30; a row past M has an offset past the resource
+  // (zeros, no memory request)
+  static_assert(NB <= 2, "activation bytes below 2^31");
   const __amdgpu_buffer_rsrc_t xrs = buffer_rsrc(x + m0 * K, static_cast<int>(2 * M * K));
   uint32_t xoff[NB][4];
 #pragma unroll

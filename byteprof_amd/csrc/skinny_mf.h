@@ -5,9 +5,10 @@
 // Operand layout (v_mfma_f32_16x16x32_bf16: A 16 x 32, B 32 x 16, D 16 x 16; lane l holds A row l % 16 and B column
 // l % 16 at K slots 8 (l / 16) .. + 7, and D rows 4 (l / 16) .. + 3 of column l % 16):
 //   - a row block is 8 consecutive weight rows; a K segment is 128 bytes of each row (64 bf16 / 128 int8 weights);
-//   - one 16-byte load per lane reads a whole segment of a block: lane (g = l / 16, i = l % 16) reads bytes
-//     16 (2 g + h) .. + 15 of row i % 8, h = i / 8, so each row is one full 128-byte line per load instruction (the
-//     rate of 1 KiB-per-row streaming; 16 rows x 64 bytes per instruction streams ~40% slower);
+//   - one 16-byte load per lane reads a whole segment of a block, each row one full 128-byte line (the rate of
+//     1 KiB-per-row streaming; 16 rows x 64 bytes per instruction streams ~40% slower). Lane (g = l / 16, i = l % 16) takes
+//     bytes 16 (2 g + h) .. + 15 of row i % 8, h = i / 8, as its operand: loaded so (MfInOrder), or loaded a row after the
+//     other (lane l: row l / 8, piece l % 8) and exchanged in LDS (MfPatch, below);
 //   - A row i of the MFMA is then weight row i % 8 restricted to half h of the segment's K slots, and B column j is
 //     activation row 8 b + j % 8 (b: the 8-row activation block) restricted to half j / 8; the lane's A and B slots
 //     cover the same K indices, so D[i][j] is a partial dot product exactly when i / 8 == j / 8: D[r][m] (half 0)
@@ -203,13 +204,14 @@ __device__ __forceinline__ void mf_wait_vm() {
   __builtin_amdgcn_s_waitcnt((n & 0xF) | ((n >> 4) << 14) | (0x7 << 4) | (0xF << 8));
 }
 
-// What turns a loaded 16 bytes of weights into the lane's MFMA operand. MfInOrder: nothing (the load was in operand order:
-// lane (g, i) reads row i % 8, piece 2 g + i / 8). MfPatch: the load was in memory order (lane l reads row l / 8, piece
-// l % 8, eight neighbouring lanes one 128-byte line) and goes through the wave's own 1 KiB LDS patch: a load whose
+// What turns a loaded 16 bytes of weights into the lane's MFMA operand. MfInOrder: nothing (the load was in operand
+// order: lane (g, i) reads row i % 8, piece 2 g + i / 8). MfPatch: the load was in memory order (lane l reads row l / 8,
+// piece l % 8, eight neighbouring lanes one 128-byte line) and goes through the wave's own 1 KiB LDS patch: a load whose
 // neighbouring lanes are in different rows takes the address unit four times as long, about 64 cycles a KiB, and a CU
 // that took its weights and activations so was bound by that, not by memory (2048 x 8192 bf16 at one row took 8.3 us from
-// memory and 8.2 from the caches; in memory order 7.8; at 8 rows 10.9 and 9.3). Piece p of row r lies at p ^ (r & 6), so that neither the
-// row-wise writes nor the operand reads conflict; the wave's LDS operations run in order, so no barrier is needed.
+// memory and 8.2 from the caches; in memory order 7.8; at 8 rows 10.9 and 9.3). Piece p of row r lies at p ^ (r & 6), so
+// that neither the row-wise writes nor the operand reads conflict; the wave's LDS operations run in order, so no barrier
+// is needed.
 struct MfInOrder {
   MfInOrder() = default;
   __device__ __forceinline__ MfInOrder(const uint8_t*, int) {}

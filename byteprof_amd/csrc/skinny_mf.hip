@@ -186,7 +186,8 @@ int mf_launch(int wkind, const void* x, const void* w, const void* scale, int sc
     if (prologue->kind != BP_PRO_UNIT_RMS && prologue->kind != BP_PRO_NORM) return BP_E_INVALID_ARG;
     if (prologue->kind == BP_PRO_NORM && prologue->gamma == nullptr) return BP_E_INVALID_ARG;
     // gamma, the residual and xout are read / written in 16-byte pieces
-    if (reinterpret_cast<uintptr_t>(prologue->gamma) % 16 != 0 || reinterpret_cast<uintptr_t>(prologue->residual) % 16 != 0 ||
+    if (reinterpret_cast<uintptr_t>(prologue->gamma) % 16 != 0 ||
+        reinterpret_cast<uintptr_t>(prologue->residual) % 16 != 0 ||
         reinterpret_cast<uintptr_t>(prologue->xout) % 16 != 0 || reinterpret_cast<uintptr_t>(prologue->gamma2) % 16 != 0)
       return BP_E_INVALID_ARG;
     if (prologue->gamma2 != nullptr && prologue->kind != BP_PRO_NORM) return BP_E_INVALID_ARG;

@@ -171,8 +171,9 @@ namespace {
 // activation operand is loaded from memory with its weights. Same operands either way: the results are equal bit
 // for bit. PRO (XL, split 1 only): a transform of the staged rows before the matmul (mf_prologue); for
 // BP_PRO_NORM, gamma and the residual rows are loaded into LDS ahead of the weights too where the launch sized the
-// LDS for them (pro.gl: 2 K (1 + rows) more bytes, always at one row, else within 80 KiB in all). NSEG > 0 (VEC only): every wave of the launch has exactly NSEG segments (the
-// host checks K / (segment x split x waves) == NSEG), run as straight-line code (MfFixed); 0: any count (MfMain).
+// LDS for them (pro.gl: 2 K (1 + rows) more bytes, always at one row, else within 80 KiB in all).
+// NSEG > 0 (VEC only): every wave of the launch has exactly NSEG segments (the host checks
+// K / (segment x split x waves) == NSEG), run as straight-line code (MfFixed); 0: any count (MfMain).
 // WR > 1 (XL only, no prologue): WR row groups of 8 RB rows, each with its own WAVES waves splitting K as above, over
 // the one LDS copy of the activation rows: the workgroup reads its activation operands once for 8 RB WR rows (the
 // bytes per weight row fall by WR), every row's sum in the same order as with WR = 1.

@@ -1,4 +1,4 @@
-// The matrix-core skinny matmul for 9..64 activation rows: the sums of skinny_mf.h (same K segments, same halves, same
+// The matrix-core skinny matmul from 9 activation rows on: the sums of skinny_mf.h (same K segments, same halves, same
 // waves, same order, so the same bits), with full MFMA tiles and coalesced operand loads.
 //
 // skinny_mf.h carries the two halves of a segment's K slots in one 16 x 16 tile (8 weight rows x 8 activation rows x 2

@@ -1,4 +1,4 @@
-// Kernels of the matrix-core skinny matmul at 9..64 activation rows (skinny_wide.h). Launched by skinny_mf.hip.
+// Kernels of the matrix-core skinny matmul from 9 activation rows on (skinny_wide.h). Launched by skinny_mf.hip.
 //
 // Reference semantics: byteprof/optim/skinny.py:36-90, via skinny_mm (skinny.py:136-166).
 
@@ -72,8 +72,9 @@ __global__ __launch_bounds__(WAVES* kWave, 2) void skinny_wide_kernel(const uint
       __builtin_amdgcn_readfirstlane(first < s_hi ? (static_cast<int>(s_hi) - first + WAVES - 1) / WAVES : 0);
 
   // the workgroup's weight rows and the activation rows as buffer resources; rows past N or M and segments past the
-  // wave's last have offsets past them (zeros, no memory request). K < 2^24: 16 RP rows x K x 2 bytes <= 2^31 - 1 by
-  // the launch's choice of RP.
+  // wave's last have offsets past them (zeros, no memory request). K is a multiple of 64 below 2^24 (the launches'
+  // kMaxVecK), so 64 rows x K x 2 bytes stay below 2^31.
+  static_assert(RP <= 4 && MB <= 4, "operand sizes below 2^31 bytes");
   const int64_t rows = std::min<int64_t>(16 * RP, N - n0);
   const __amdgpu_buffer_rsrc_t wrs = buffer_rsrc(w + n0 * K * G::kEB, static_cast<int>(rows * K * G::kEB));
   const __amdgpu_buffer_rsrc_t xrs = buffer_rsrc(x + m0 * K, static_cast<int>(2 * M * K));

@@ -36,7 +36,9 @@ from . import skinny as S
 
 MAX_CACHE_LEN = 1024  # the reference's static cache length (olmo.py:16)
 ROPE_ATTENTION_ROWS = 16  # most rows of one fused q/k-norm + RoPE + cache + attention launch
-PREFILL_ROWS = 256  # most prompt rows of one pass (its buffers: about 5 (H + F) KiB a row, allocated at the first prompt)
+# Most prompt rows of one pass. Its buffers, allocated at the first prompt: 14 H + 2 F bytes a row (2048 x 8192: 45 KB, 11.5
+# MB in all), 4 F more a row without the SiLU epilogue, and the split plans' partials.
+PREFILL_ROWS = 256
 VERIFY_ROWS = 16  # rows of the verify-pass buffers (allocated once per decoder, never reallocated)
 PRO_MAX_ROWS = {"bf16": 3, "int8": 1, "int4": 1}  # most rows of a linear launch with the norm as its prologue
 INT4_PRO_LDS_BYTES = 64 * 1024  # the int4 kernel's norm prologue: rows, gamma, residual rows, gamma2, (2 M + 2) K bf16
@@ -455,7 +457,7 @@ class OlmoDecoder:
     def prefill(self, ids: torch.Tensor) -> None:
         """The prompt ids [L] at positions 0 .. L - 1: fills the caches, leaves the last position's logits in `logits`,
         the first new token in tok and L in pos, bit for bit as L calls of step() from position 0 would. Passes of up to
-        PREFILL_ROWS rows: 160 positions of the OLMo-2-1B shape in one (9 launches a layer) instead of 160 steps of 83
+        PREFILL_ROWS rows: 160 positions of the OLMo-2-1B shape in one (8 launches a layer) instead of 160 steps of 83
         launches. After the last layer's cache write only the prompt's last row goes on."""
         length = ids.shape[0]
         self.pos.zero_()

@@ -5,11 +5,12 @@ Drop-in for byteprof/optim/skinny.py: same names (`skinny_mm`, `get_cfg`, `_bm`,
 bf16 activations, fp32 accumulation, bf16 output; weights bf16 [N, K], int8 [N, K] with one scale per output row
 (bf16, fp16 or fp32), or int4 group-128 in the reference's tile-major format.
 
-bf16 and int8 run on one matrix-core kernel family for every row count (csrc/skinny_mf.h, csrc/skinny_wide.h past 8 rows):
-one launch takes up to MAX_M = 64 activation rows and streams every weight byte once; the K order of every sum depends only on the shape's
-(waves, split), never on M, so output row i is bitwise the same whether it is computed alone or with up to 63 other
-rows (the reference's row-independence contract, test_skinny.py:110-120, here over M = 1..64). int4 runs on
-skinny_int4.hip and skinny_int4_wide.hip (their order ignores M too).
+bf16 and int8 run on one matrix-core kernel family for every row count (csrc/skinny_mf.h up to 8 rows, csrc/skinny_wide.h
+past 16, in between by the number of weight rows): one launch takes up to MAX_M = 64 activation rows and streams every
+weight byte once; the K order of every sum depends only on the shape's (waves, split), never on M, so output row i is
+bitwise the same whether it is computed alone or with up to 63 other rows (the reference's row-independence contract,
+test_skinny.py:110-120, here over M = 1..64). int4 runs on skinny_int4.hip and skinny_int4_wide.hip (their order ignores
+M too).
 
 `cfg` is (rows, waves, split) for the bf16 / int8 kernel (rows: weight rows per workgroup, a multiple of 8;
 waves: wavefronts sharing a workgroup's K range; split: K ranges in separate workgroups, added in fixed order) or
@@ -20,7 +21,6 @@ reference forced by raw-pointer kernels: x must be bfloat16 and on the GPU, w, s
 from __future__ import annotations
 
 import ctypes
-
 import functools
 import json
 from pathlib import Path
@@ -35,7 +35,7 @@ ROWS_PER_LAUNCH = MAX_M
 
 _KIND_CODE = {"bf16": 0, "int8": 1}
 XS_STAGE, XS_GENERAL = 1, 2  # BP_XS_STAGE, BP_XS_GENERAL: activations staged in LDS; the general segment loop
-XS_ROWS2, XS_ROWS4 = 4, 8     # BP_XS_ROWS2 / 4: with XS_STAGE at 9..16 rows, 2 / 4 row groups over one staged copy
+XS_ROWS2, XS_ROWS4 = 4, 8  # BP_XS_ROWS2 / 4: with XS_STAGE at 9..16 rows, 2 / 4 row groups over one staged copy
 XS_ROWS = XS_ROWS2 | XS_ROWS4
 _RB_MENU = (1, 2, 4)        # 8-row weight blocks per workgroup
 _WAVES_MENU = (1, 2, 4, 8)
@@ -102,7 +102,8 @@ def _default_waves(kind: str, n: int, k: int) -> int:
 
 def _default_rb(kind: str, n: int, k: int, m: int) -> int:
     """8-row weight blocks per workgroup at m rows: each activation operand serves 8 times as many weight rows, but there
-    are as many fewer workgroups. Past 8 rows the launch picks its own tile.
+    are as many fewer workgroups. Past 8 rows the wide kernel picks its own tile, and where it does not run (few weight
+    rows) one block is the fastest.
 
     Up to 2560 weight rows 1 (2048 x 4096 bf16 at 5 rows 5.2, with two 6.4). int8: 2 (4096 x 8192 at one row 8.9, 9.3 with
     one and 12.8 with four; 16000 x 4096 at 5 rows 15.4, 17.4, 16.6), 4 at 6..8 rows of 4608 to 8192 (8192 x 14336 at 8 rows
@@ -130,8 +131,8 @@ def _default_split(kind: str, n: int, k: int, waves: int) -> int:
     over few weight rows: from 160 segments (int8: 112) on, while a wave keeps four and the first launch has fewer than
     192 workgroups (bf16 at 16 rows without / with: 64 x 32768 36 / 10.6 (8 ranges), 300 x 14336 19 / 9.7 (4); int8 64 x
     32768 26 / 9.9; at one row 13.3 / 6.9, 7.9 / 6.3, 10.9 / 6.7), and for bf16 at 32 segments a wave up to 512 (2048 x
-    32768 at one row 26.7 / 27.4, at 16 rows 43 / 30). Below that the plain launch is the faster one up to 8 rows (512 x 8192 bf16
-    5.1 and 5.6; 1920 x 7168 6.8 and 9.1; 300 x 1024 2.6 and 4.4), though not at 16 (512 x 8192 11.2 and 8.1).
+    32768 at one row 26.7 / 27.4, at 16 rows 43 / 30). Below that the plain launch is the faster one up to 8 rows (512 x
+    8192 bf16 5.1 and 5.6; 1920 x 7168 6.8 and 9.1; 300 x 1024 2.6 and 4.4), though not at 16 (512 x 8192 11.2 and 8.1).
 
     A K off the segments takes the element loads (4 waves, one segment in flight), where a segment costs a wave 1 to 2 us:
     past eight segments a wave the split grows while a wave keeps two (four past 8 ranges: the reduce reads every range)

@@ -13,12 +13,12 @@ loop), and at one row with a norm prologue (split 1). It keeps the fastest one-r
 split > 1 must win by more than 3%; when that order has no split, the split-1 order within 5% of it whose plain and
 prologue launches are fastest together (the decode step runs the prologue form); then, among the orders within 2%
 of that, the fastest at 16 rows. Then, at that K order, it picks the weight blocks per workgroup and
-the flags for each bucket whose launches use them (1; 8: four and eight rows together; 16: nine and sixteen, the row groups over
-one staged copy among its plans). The wide kernel picks its own tile and ignores both: the buckets of its launches (all
-past 16 rows) are timed once and hold rb 1, xs 0 (`--plans-only 16` retunes just those buckets in an existing table; for int4 it times the
-entry's plan again). Last, for
-launches with a norm prologue (bp_skinny_mf_pro: the decode loops' q|k|v, gate|up and LM head launches), the weight
-blocks per workgroup at the same K order, for buckets 1 and 8 (rb_pro; `--pro-only` retunes just those).
+the flags for each bucket whose launches use them (1; 8: four and eight rows together; 16: nine and sixteen, the row
+groups over one staged copy among its plans). The wide kernel picks its own tile and ignores both: the buckets of its
+launches (all past 16 rows) are timed once and hold rb 1, xs 0 (`--plans-only 16` retunes just those buckets in an
+existing table; for int4 it times the entry's plan again). Last, for launches with a norm prologue (bp_skinny_mf_pro:
+the decode loops' q|k|v, gate|up and LM head launches), the weight blocks per workgroup at the same K order, for
+buckets 1 and 8 (rb_pro; `--pro-only` retunes just those).
 
 Usage: python -m byteprof_amd.tune [--shapes N:K,...] [--kinds bf16,int8,int4] [--out path] [--pro-only]
                                    [--plans-only BUCKETS]
@@ -130,7 +130,8 @@ def _best_plan(kind, ring, x, y, waves, split, rows_list) -> tuple[float, int, i
     kernel, one plan stands for all."""
     best = None
     if all(_wide(kind, m, y.shape[1], x.shape[1], waves, split) for m in rows_list):
-        return sum(_time_calls(_launcher(kind, ring, x[:m].contiguous(), y[:m], 1, waves, split, 0)) for m in rows_list), 1, 0
+        times = [_time_calls(_launcher(kind, ring, x[:m].contiguous(), y[:m], 1, waves, split, 0)) for m in rows_list]
+        return sum(times), 1, 0
     for rb, xs in _plans(kind, max(rows_list), x.shape[1], waves, split):
         t = sum(_time_calls(_launcher(kind, ring, x[:m].contiguous(), y[:m], rb, waves, split, xs))
                 for m in rows_list)
@@ -384,8 +385,8 @@ def main(argv=None) -> int:
                        "(bf16, int8): waves and split of the matrix-core kernel (they fix the K order for every row "
                        "count), rb = 8-row weight blocks per workgroup and xs = xstage flags (1: activations "
                        "staged in LDS, 2: the general segment loop instead of the straight-line kernel of the "
-                       "segment count), per row bucket (1, 8, 16, 32, 64; the wide kernel, past 16 rows always, ignores both: "
-                       "1 and 0 there), rb_pro = rb of launches with a norm "
+                       "segment count), per row bucket (1, 8, 16, 32, 64; the wide kernel, past 16 rows always, "
+                       "ignores both: 1 and 0 there), rb_pro = rb of launches with a norm "
                        "prologue (buckets 1 and 8), us = measured time per call by row count (ring of distinct "
                        "weights, HIP graph); int4|N|K: tile_rows = the rows per tile to pack the weight "
                        "with, waves and split of the int4 kernel at those tile rows, us per row count, and tiles = the "

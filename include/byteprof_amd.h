@@ -53,10 +53,10 @@ size_t bp_skinny_workspace_bytes(int64_t M, int64_t N, int split);
  *   BP_DT_BF16 / F16 / F32 on the fp32 sum), 1 <= M <= 64 per call (M = 0 or N = 0: no-op; K = 0: zeros).
  * One load instruction reads a 128-byte segment of 8 consecutive weight rows (one full line per row); the
  * activations are the MFMA's B operand (8 activation rows per 16 columns, the other 8 columns carry the other half of
- * the segment's K slots); from 9 to 17 rows on (by sizes) a kernel with 16 x 16 blocks takes over (bp_skinny_mf_wide), which picks its
- * own tile and ignores rb and xstage. Tile configuration: rb = 8-row weight blocks per workgroup (1, 2, 4; 4 up to
- * M = 16), waves = wavefronts sharing the workgroup's K segments (1, 2, 4, 8; segment s to wave s % waves), split = K ranges
- * in separate workgroups whose fp32 partials are added in split order by a second kernel (workspace as for
+ * the segment's K slots); from 9 to 17 rows on (by sizes) a kernel with 16 x 16 blocks takes over (bp_skinny_mf_wide),
+ * which picks its own tile and ignores rb and xstage. Tile configuration: rb = 8-row weight blocks per workgroup (1, 2, 4;
+ * 4 up to M = 16), waves = wavefronts sharing the workgroup's K segments (1, 2, 4, 8; segment s to wave s % waves), split =
+ * K ranges in separate workgroups whose fp32 partials are added in split order by a second kernel (workspace as for
  * bp_skinny_workspace_bytes), xstage: flags BP_XS_STAGE (each workgroup copies its activation rows and K range to
  * LDS first; up to M = 16 and bp_skinny_mf_stage_bytes() >= 0; else the activation operands are loaded with the
  * weights) and BP_XS_GENERAL (the general segment loop; without it, a launch whose waves have exactly 4, 8 or 16
@@ -64,10 +64,10 @@ size_t bp_skinny_workspace_bytes(int64_t M, int64_t N, int split);
  * BP_XS_ROWS4 make the workgroup 2 / 4 row groups of rb blocks, each with its own `waves` waves, over one LDS copy of
  * the activation rows (the activation bytes per weight row fall 2 / 4x; up to 64 KiB of LDS,
  * bp_skinny_mf_stage_bytes_rows(); waves x groups <= 16; not with 16 segments a wave). The K order of every sum
- * depends only on (K, waves, split): output row i is bitwise independent of M (1..64), rb and xstage. K not a multiple of the 128-byte segment
- * (64 bf16 / 128 int8 elements), x, w not 16-byte aligned, or K >= 2^24 (the vector loads read the activations
- * through one buffer resource, under 2^31 bytes at 64 rows): an element-load variant with the same segments (rb 1,
- * 4 waves, xstage 0).
+ * depends only on (K, waves, split): output row i is bitwise independent of M (1..64), rb and xstage. K not a multiple of
+ * the 128-byte segment (64 bf16 / 128 int8 elements), x, w not 16-byte aligned, or K >= 2^24 (the vector loads read the
+ * activations through one buffer resource, under 2^31 bytes at 64 rows): an element-load variant with the same segments
+ * (rb 1, 4 waves, xstage 0).
  * Replaces: byteprof/optim/skinny.py:36-90 (_skinny_kernel MODE 0 / 1, _split_reduce) and :111-133 (_launch) via
  *           skinny_mm (skinny.py:136-166) for every BM bucket (16, 32, 64); at M = 1 with int8 weights, the one-row
  *           int8 product byteprof/quant/triton_int8.py:16-47 (_gemv_int8, gemv_int8).
@@ -132,8 +132,8 @@ int bp_skinny_mf_static(int wkind, const void* x, const void* w, const void* sca
  *                    plain norm), bit for bit bp_decode_norm_residual's output (its summation order), so that the
  *                    norm of a sublayer's output and the residual add run inside the next linear;
  * and when xout is not NULL the transformed rows [M, K] are written there (by one workgroup; an xout whose M x K
- * elements overlap those of x or of residual is refused with BP_E_INVALID_ARG before anything is enqueued). With gamma2 (BP_PRO_NORM only) the matmul reads bf16(gamma2 * (t * (1 / sqrt(mean(t^2) + eps))))
- * of those rows t instead (xout still receives t): a decoder's last post-feed-forward norm and its final norm in the
+ * elements overlap those of x or of residual is refused with BP_E_INVALID_ARG before anything is enqueued). With gamma2
+ * (BP_PRO_NORM only) the matmul reads bf16(gamma2 * (t * (1 / sqrt(mean(t^2) + eps)))) of those rows t instead (xout still receives t): a decoder's last post-feed-forward norm and its final norm in the
  * LM head's launch, bit for bit bp_decode_norm_residual followed by the BP_PRO_NORM launch. gamma, residual, xout
  * and gamma2 16-byte aligned. BP_PRO_NORM keeps gamma, the residual rows and gamma2 in LDS
  * beside the staged rows at one row, and at more rows while all of it fits 80 KiB (else it reads them from memory;
